@@ -126,6 +126,62 @@ def test_q4_matmul_weight_operand_bit_exact(exe, huge):
     assert np.array_equal(got, ref), int(np.sum(got != ref))
 
 
+# The K-splitting kernels of few rows at the edges of their tiles: 32-row tiles
+# (1, 31, 32, 33 rows; one to sixteen K units for 8 waves), 64-row tiles (from
+# 256 tiles of 32 rows on) and 64 x 128 tiles with K in two sets (from 256 tiles
+# of 64 x 32 on, K a multiple of 512), and T = 300 of K = 768, which that one
+# does not take.
+@pytest.mark.parametrize("T,in_f,out_f", [(1, 256, 128), (31, 2048, 128), (33, 768, 256), (32, 4096, 128),
+                                          (37, 2048, 5120), (65, 2304, 5120), (129, 2048, 5120), (333, 512, 5120),
+                                          (300, 768, 5120), (1000, 4096, 2048)])
+def test_q4_matmul_few_rows(exe, T, in_f, out_f):
+    """5e-3 against the kernel's bf16 operands in fp64: the fp32 sums differ by
+    1e-6, the bf16 output by half a step (2^-9)."""
+    rng = np.random.default_rng(7100 + T + in_f)
+    w, s, b = synth.centered_quant(rng, out_f, in_f)
+    X = synth.bf16_normal(rng, (T, in_f))
+    pad = exe.alloc((T + 1, out_f), np.uint16)
+    pad.upload(np.full((T + 1, out_f), 0x1234, np.uint16))  # the row past T must stay
+    exe.q4_matmul(exe.upload(w), exe.upload(s), exe.upload(b), exe.upload(X), pad, T, in_f, out_f, 64)
+    got = pad.download()
+    assert np.all(got[T] == 0x1234)
+    W = synth.bf16_bits_to_f32(synth.f32_to_bf16_bits(O.dequant(4, w, s, b, out_f, in_f)))
+    _close(_f32(got[:T]), (_f32(X) @ W.astype(np.float64).T), 5e-3)
+
+
+@pytest.mark.parametrize("T,in_f,out_f,huge", [(64, 2048, 5120, False), (64, 2048, 5120, True),
+                                               (200, 2048, 5120, False), (200, 2048, 5120, True)])
+def test_q4_matmul_few_rows_operand_bit_exact(exe, T, in_f, out_f, huge):
+    """As test_q4_matmul_weight_operand_bit_exact (which takes the 32-row
+    kernel), for the 64-row and the K-in-two kernels: row t is one-hot at column
+    (37 t) % in_f, so Y[t] is that column of the bf16 weight operand."""
+    rng = np.random.default_rng(4300 + T + huge)
+    w = rng.integers(0, 2**32, size=(out_f, in_f // 8), dtype=np.uint64).astype(np.uint32)
+    s, b = _extreme_scales(rng, out_f, in_f // 64, huge)
+    cols = 37 * np.arange(T) % in_f
+    X = np.zeros((T, in_f), np.uint16)
+    X[np.arange(T), cols] = 0x3F80  # bf16 1.0
+    Y = exe.alloc((T, out_f), np.uint16)
+    exe.q4_matmul(exe.upload(w), exe.upload(s), exe.upload(b), exe.upload(X), Y, T, in_f, out_f, 64)
+    ref = synth.f32_to_bf16_bits(O.dequant(4, w, s, b, out_f, in_f))[:, cols].T
+    got = Y.download()
+    assert np.array_equal(got, ref), int(np.sum(got != ref))
+
+
+def test_q4_matmul_scales_at_two_byte_alignment(exe):
+    """Scales and biases that are not 8-byte aligned keep the 128-row tiles,
+    with the same result to the rounding of their sums' order."""
+    T, in_f, out_f = 40, 2048, 768
+    rng = np.random.default_rng(4400)
+    w, s, b = synth.centered_quant(rng, out_f, in_f)
+    X = exe.upload(synth.bf16_normal(rng, (T, in_f)))
+    dw, y0, y1 = exe.upload(w), exe.alloc((T, out_f), np.uint16), exe.alloc((T, out_f), np.uint16)
+    exe.q4_matmul(dw, exe.upload(s), exe.upload(b), X, y0, T, in_f, out_f, 64)
+    off = [exe.upload(np.concatenate([np.zeros(1, np.uint16), a.reshape(-1)])) for a in (s, b)]
+    exe.q4_matmul(dw, off[0].ptr + 2, off[1].ptr + 2, X, y1, T, in_f, out_f, 64)
+    _close(_f32(y1.download()), _f32(y0.download()), 2e-3, 1e-2)
+
+
 @pytest.mark.parametrize("T,seed", [(64, 0), (37, 1), (1, 2)])
 def test_moe_prefill_zipf_vs_oracle(exe, qwen, T, seed):
     t, layer, L = qwen
