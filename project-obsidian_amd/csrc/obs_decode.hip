@@ -5,193 +5,258 @@
 // The reference pages the 8 selected experts off SSD into a pool
 // (disk_io.rs:79-102, forward.rs:431-435) and issues 5 dispatches per expert;
 // here the whole expert table is resident in HBM (stacked [E, ...] tensors)
-// and the layer runs as 4 launches: gate logits, top-k, gate/up+SwiGLU,
-// down+combine. Weights are read exactly once with 16-byte coalesced loads.
+// and the layer runs as 3 launches: router (with the post-attention norm),
+// gate/up+SwiGLU, down+combine (two or three more where the router is not one
+// launch). Weights are read exactly once with 16-byte coalesced loads.
 //
 // Numerics: dots accumulate in fp32 using the per-group factored form
 //   sum_c (q_c*s + b) * x_c = s * sum_c q_c*x_c + b * sum_c x_c
 // (exact algebra; it removes one multiply-add per weight). h stays fp32,
-// the combine accumulates sum_r w_r*y_r in fp32 in rank order (forward.rs:440
-// order) and rounds once to bf16.
-#include "obs_internal.hpp"
+// the combine accumulates sum_r w_r*y_r in fp32 (forward.rs:440) and rounds
+// once to bf16.
+#include "obs_q4_dequant.hpp"
 
 namespace obs {
 int check_router_shape(obs_ctx* ctx, const char* who, uint32_t in, uint32_t n_exp, uint32_t group);
-int launch_route(obs_ctx* ctx, const uint32_t* w8, const uint16_t* s, const uint16_t* b, const uint16_t* x,
-                 float* logits, int32_t* ids, float* w, uint32_t T, uint32_t in, uint32_t n_exp, uint32_t group,
-                 uint32_t k, int norm_topk, int rule);
 }  // namespace obs
 
 namespace {
 
 using namespace obsd;
 
-constexpr int GU_ROWS_PER_WAVE = 2;
-constexpr int GU_WAVES = 4;
-constexpr int DN_ROWS_PER_WAVE = 2;
-constexpr int DN_WAVES = 4;
-
-// h[r, o] = silu(gate_e[o] . x) * (up_e[o] . x) for e = ids[r].
-// One wave per (r, o) row pair; lane l owns the 8*WPL contiguous columns
-// [l*8*WPL, (l+1)*8*WPL), which lie inside one quantization group.
-template <int WPL>
-__global__ void __launch_bounds__(GU_WAVES * 64) decode_gateup_kernel(
-    const uint32_t* __restrict__ gw, const uint16_t* __restrict__ gs, const uint16_t* __restrict__ gb,
-    const uint32_t* __restrict__ uw, const uint16_t* __restrict__ us, const uint16_t* __restrict__ ub,
-    const uint16_t* __restrict__ x, const int32_t* __restrict__ ids, float* __restrict__ h,
-    uint32_t n_exp, uint32_t k, uint32_t H, uint32_t I, uint32_t group) {
-  constexpr int C = 8 * WPL;
-  const uint32_t lane = threadIdx.x & 63;
-  const uint32_t wave = blockIdx.x * GU_WAVES + threadIdx.x / 64;
-  // x chunk and its sum, once per wave
-  float xf[C];
-  const uint16_t* xr = x + lane * C;
+// A lane's share of a packed row: CH chunks of W words (8 columns each), chunk i
+// at word W * (lane + 64 i), so a wave reads a row in whole, contiguous runs.
+template <int W, int CH>
+__device__ __forceinline__ void load_words(const uint32_t* row, uint32_t lane, uint32_t (&q)[W * CH]) {
 #pragma unroll
-  for (int c = 0; c < C; c += 8) {
-    const uint4 v = *reinterpret_cast<const uint4*>(xr + c);
-    xf[c + 0] = bf16lo(v.x); xf[c + 1] = bf16hi(v.x);
-    xf[c + 2] = bf16lo(v.y); xf[c + 3] = bf16hi(v.y);
-    xf[c + 4] = bf16lo(v.z); xf[c + 5] = bf16hi(v.z);
-    xf[c + 6] = bf16lo(v.w); xf[c + 7] = bf16hi(v.w);
-  }
-  float xs = 0.0f;
-#pragma unroll
-  for (int c = 0; c < C; ++c) xs = xs + xf[c];
-  const uint32_t words = H / 8, groups = H / group;
-  const uint32_t g = (lane * C) / group;
-#pragma unroll
-  for (int rr = 0; rr < GU_ROWS_PER_WAVE; ++rr) {
-    const uint32_t row = wave * GU_ROWS_PER_WAVE + rr;  // r * I + o
-    if (row >= k * I) break;
-    const uint32_t r = row / I, o = row % I;
-    const int32_t e = ids[r];
-    float hv = 0.0f;
-    if (e >= 0 && static_cast<uint32_t>(e) < n_exp) {
-      const uint64_t wrow = (static_cast<uint64_t>(e) * I + o);
-      const uint32_t* gp = gw + wrow * words + lane * WPL;
-      const uint32_t* up = uw + wrow * words + lane * WPL;
-      uint32_t gq[WPL], uq[WPL];
-      if constexpr (WPL % 4 == 0) {
-#pragma unroll
-        for (int j = 0; j < WPL; j += 4) {
-          const uint4 a = *reinterpret_cast<const uint4*>(gp + j);
-          const uint4 c = *reinterpret_cast<const uint4*>(up + j);
-          gq[j] = a.x; gq[j + 1] = a.y; gq[j + 2] = a.z; gq[j + 3] = a.w;
-          uq[j] = c.x; uq[j + 1] = c.y; uq[j + 2] = c.z; uq[j + 3] = c.w;
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < WPL; j += 2) {
-          const uint2 a = *reinterpret_cast<const uint2*>(gp + j);
-          const uint2 c = *reinterpret_cast<const uint2*>(up + j);
-          gq[j] = a.x; gq[j + 1] = a.y;
-          uq[j] = c.x; uq[j + 1] = c.y;
-        }
-      }
-      const uint64_t srow = wrow * groups + g;
-      const float sg = bf16_to_f32(gs[srow]), bgv = bf16_to_f32(gb[srow]);
-      const float su = bf16_to_f32(us[srow]), bu = bf16_to_f32(ub[srow]);
-      float ag = 0.0f, au = 0.0f;
-#pragma unroll
-      for (int j = 0; j < WPL; ++j) {
-        ag = dot8_q4(gq[j], xf + 8 * j, ag);
-        au = dot8_q4(uq[j], xf + 8 * j, au);
-      }
-      float pg = __builtin_fmaf(sg, ag, bgv * xs);
-      float pu = __builtin_fmaf(su, au, bu * xs);
-      pg = wave_sum_asc(pg);
-      pu = wave_sum_asc(pu);
-      hv = silu_mul(pg, pu);
+  for (int i = 0; i < CH; ++i) {
+    const uint32_t* p = row + W * (lane + 64u * i);
+    if constexpr (W == 4) {
+      const uint4 v = load_stream(p);
+      q[4 * i] = v.x; q[4 * i + 1] = v.y; q[4 * i + 2] = v.z; q[4 * i + 3] = v.w;
+    } else {
+      const uint2 v = *reinterpret_cast<const uint2*>(p);
+      q[2 * i] = v.x; q[2 * i + 1] = v.y;
     }
-    if (lane == 0) h[row] = hv;
   }
 }
 
+// Sums of q_j * x_j over the 8 nibbles of w: even nibbles as the f16 subnormals
+// q * 2^-24, odd ones as q * 2^-20 (masked in place), each converted exactly
+// inside an fp32 fma. 13 instructions instead of dot8_q4's 19; the caller puts
+// the powers of two back (dot_mix_sum), which is exact.
+struct DotMix {
+  float a24, a20;
+};
+__device__ __forceinline__ void dot8_q4_mix(uint32_t w, const float* x, DotMix& d) {
+  const uint32_t w8 = w >> 8;
+  const uint32_t p04 = w & 0x000F000Fu, p15 = w & 0x00F000F0u, p26 = w8 & 0x000F000Fu, p37 = w8 & 0x00F000F0u;
+  d.a24 = fma_mix_f16<0>(p04, x[0], d.a24);
+  d.a20 = fma_mix_f16<0>(p15, x[1], d.a20);
+  d.a24 = fma_mix_f16<0>(p26, x[2], d.a24);
+  d.a20 = fma_mix_f16<0>(p37, x[3], d.a20);
+  d.a24 = fma_mix_f16<1>(p04, x[4], d.a24);
+  d.a20 = fma_mix_f16<1>(p15, x[5], d.a20);
+  d.a24 = fma_mix_f16<1>(p26, x[6], d.a24);
+  d.a20 = fma_mix_f16<1>(p37, x[7], d.a20);
+}
+__device__ __forceinline__ float dot_mix_sum(const DotMix& d) {
+  return __builtin_fmaf(d.a20, 0x1p20f, d.a24 * 0x1p24f);
+}
+
+constexpr uint32_t GU_WAVES = 4;
+constexpr uint32_t GU_WAVES_MAX = 2048;  // waves a gate/up launch aims at: 8 per CU
+
+// h[r, o] = silu(gate_e[o] . x) * (up_e[o] . x) for e = ids[r], one wave per PR
+// consecutive (r, o) row pairs; lane l owns the 8*W columns of CH chunks (as
+// load_words), each inside one quantization group. H = 512 * W * CH.
+//
+// Bound by HBM: k * I * H weights of both matrices at 4.5 bits. Every wave
+// requests all of its rows at once (6 row pairs of H = 4096 are 24 KB a wave, 196
+// KB in flight per CU) and there is no second round of waves, so the first rows'
+// dots run while the last are on their way; twice the waves of 3 rows measured
+// 20.1 us against 18.3. E 16, H 4096, I 2048, k 6 (57 MB): 20.3 us with 2 rows a
+// wave, 22.2 with 6 and dot8_q4 over 64 contiguous columns a lane, 18.3 us (3.1
+// TB/s) as it is.
+// NORM: x is normalised first, in obs_rmsnorm's sequence (its sum of squares over
+// the columns a lane owns there), so no launch of its own is needed (4.6 us).
+template <int W, int CH, int PR, bool NORM>
+__global__ void __launch_bounds__(GU_WAVES * 64, 2) decode_gateup_kernel(
+    const uint32_t* __restrict__ gw, const uint16_t* __restrict__ gs, const uint16_t* __restrict__ gb,
+    const uint32_t* __restrict__ uw, const uint16_t* __restrict__ us, const uint16_t* __restrict__ ub,
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ norm_w, float eps, const int32_t* __restrict__ ids,
+    float* __restrict__ h, uint32_t n_exp, uint32_t k, uint32_t I) {
+  constexpr uint32_t C = 8 * W, H = 64 * C * CH, GROUP = 64, words = H / 8, groups = H / GROUP;
+  constexpr uint32_t XQ = CH * C / 8;  // 16-byte pieces of a lane's share of x
+  const uint32_t lane = threadIdx.x & 63;
+  const uint32_t row0 = __builtin_amdgcn_readfirstlane((blockIdx.x * GU_WAVES + threadIdx.x / 64u) * PR);
+  const uint32_t rows = k * I;
+  if (row0 >= rows) return;  // wave-uniform
+  int32_t e[PR];
+#pragma unroll
+  for (int i = 0; i < PR; ++i) e[i] = ids[min(row0 + i, rows - 1u) / I];
+  uint4 xq[XQ], nq[XQ], xn[XQ];
+#pragma unroll
+  for (uint32_t j = 0; j < XQ; ++j) {
+    const uint32_t col = C * (lane + 64u * (8u * j / C)) + 8u * j % C;
+    xq[j] = *reinterpret_cast<const uint4*>(x + col);
+    if (NORM) {
+      nq[j] = *reinterpret_cast<const uint4*>(norm_w + col);
+      if (CH > 1) xn[j] = *reinterpret_cast<const uint4*>(x + CH * C * lane + 8u * j);  // the lane's columns in obs_rmsnorm
+    }
+  }
+  uint32_t gq[PR][W * CH], uq[PR][W * CH];
+  uint16_t sg[PR][CH], bg[PR][CH], su[PR][CH], bu[PR][CH];
+#pragma unroll
+  for (int i = 0; i < PR; ++i) {  // an id out of range: expert 0's rows, their sums unused
+    const uint32_t ei = static_cast<uint32_t>(e[i]) < n_exp ? static_cast<uint32_t>(e[i]) : 0u;
+    const uint64_t wrow = static_cast<uint64_t>(ei) * I + min(row0 + i, rows - 1u) % I;
+    load_words<W, CH>(gw + wrow * words, lane, gq[i]);
+    load_words<W, CH>(uw + wrow * words, lane, uq[i]);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const uint64_t srow = wrow * groups + (lane + 64u * c) * C / GROUP;
+      sg[i][c] = gs[srow];
+      bg[i][c] = gb[srow];
+      su[i][c] = us[srow];
+      bu[i][c] = ub[srow];
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);  // every load is on its way before the first wait
+  float inv = 0.0f;
+  if (NORM) {
+    float ss = 0.0f;
+#pragma unroll
+    for (uint32_t j = 0; j < XQ; ++j) {
+      const uint4 v = CH > 1 ? xn[j] : xq[j];
+      const uint32_t d[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        ss = __builtin_fmaf(bf16lo(d[p]), bf16lo(d[p]), ss);
+        ss = __builtin_fmaf(bf16hi(d[p]), bf16hi(d[p]), ss);
+      }
+    }
+    inv = 1.0f / __builtin_sqrtf(wave_sum_asc(ss) / static_cast<float>(H) + eps);
+  }
+  float xf[CH * C], xs[CH];
+#pragma unroll
+  for (uint32_t j = 0; j < XQ; ++j) {
+    const uint32_t d[4] = {xq[j].x, xq[j].y, xq[j].z, xq[j].w}, n[4] = {nq[j].x, nq[j].y, nq[j].z, nq[j].w};
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const uint32_t v = NORM ? pack_bf16x2((bf16lo(d[p]) * inv) * bf16lo(n[p]), (bf16hi(d[p]) * inv) * bf16hi(n[p])) : d[p];
+      xf[8 * j + 2 * p] = bf16lo(v);
+      xf[8 * j + 2 * p + 1] = bf16hi(v);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    xs[c] = 0.0f;
+#pragma unroll
+    for (uint32_t j = 0; j < C; ++j) xs[c] = xs[c] + xf[C * c + j];
+  }
+  float my_g = 0.0f, my_u = 0.0f;  // lane i < PR: the sums of row row0 + i
+  bool mine = false;
+#pragma unroll
+  for (int i = 0; i < PR; ++i) {
+    float pg = 0.0f, pu = 0.0f;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      DotMix ag{0.0f, 0.0f}, au{0.0f, 0.0f};
+#pragma unroll
+      for (int j = 0; j < W; ++j) {
+        dot8_q4_mix(gq[i][W * c + j], xf + C * c + 8 * j, ag);
+        dot8_q4_mix(uq[i][W * c + j], xf + C * c + 8 * j, au);
+      }
+      pg = __builtin_fmaf(bf16_to_f32(sg[i][c]), dot_mix_sum(ag), __builtin_fmaf(bf16_to_f32(bg[i][c]), xs[c], pg));
+      pu = __builtin_fmaf(bf16_to_f32(su[i][c]), dot_mix_sum(au), __builtin_fmaf(bf16_to_f32(bu[i][c]), xs[c], pu));
+    }
+    pg = wave_sum_asc(pg);
+    pu = wave_sum_asc(pu);
+    my_g = lane == static_cast<uint32_t>(i) ? pg : my_g;
+    my_u = lane == static_cast<uint32_t>(i) ? pu : my_u;
+    mine = lane == static_cast<uint32_t>(i) ? static_cast<uint32_t>(e[i]) < n_exp : mine;
+  }
+  if (lane < PR && row0 + lane < rows) h[row0 + lane] = mine ? silu_mul(my_g, my_u) : 0.0f;
+}
+
 // y[o] = (residual[o]) + sum_r w_r * (down_{e_r}[o] . h_r), one wave per output
-// row; lane l -> rank r = l/8 and column slice m = l%8 of CPL = I/8 columns.
-template <int CPL>
-__global__ void __launch_bounds__(DN_WAVES * 64) decode_down_kernel(
+// row. The k * I columns of an output row are k * I / 32 chunks (16 bytes of one
+// expert's row, half a quantization group); lane l takes chunks l, l + 64, ..., so
+// a row's weights are at most 8 whole-wave loads (NC) whatever I is.
+//
+// Bound by HBM (k * I * H weights): a wave requests all of its weights before it
+// uses the first. h is staged in LDS in the order the lanes read it
+// ([chunk / 64][float4][lane], the lane xor-ed with the float4's index so that the
+// stores of one chunk's 8 float4 spread over the banks). E 16, H 4096, I 2048, k 6
+// (28 MB): 10.1 us (11.1 with two output rows per wave, which reads h half as
+// often). A lane that kept the I / 8 values of its part of a rank's h in registers
+// spilled them from I = 1,024 on: 72.5 us.
+constexpr uint32_t DN_WAVES = 8;
+
+template <int NC>
+__global__ void __launch_bounds__(DN_WAVES * 64, 2) decode_down_kernel(
     const uint32_t* __restrict__ dw, const uint16_t* __restrict__ ds, const uint16_t* __restrict__ db,
     const float* __restrict__ h, const int32_t* __restrict__ ids, const float* __restrict__ wts,
     const uint16_t* __restrict__ residual, uint16_t* __restrict__ y, uint32_t n_exp, uint32_t k,
     uint32_t H, uint32_t I, uint32_t group) {
-  constexpr int BLK = CPL / 32;  // 32-column blocks per lane (each inside one group)
-  extern __shared__ float sh_h[];  // [k][I]
-  {
-    // stage h in batches of 8 independent 16-byte loads per thread (k*I % 4 == 0)
-    const uint32_t n4 = (k * I) / 4;
-    const float4* h4 = reinterpret_cast<const float4*>(h);
-    float4* s4 = reinterpret_cast<float4*>(sh_h);
-    for (uint32_t base = threadIdx.x; base < n4; base += 8 * blockDim.x) {
-      float4 v[8];
+  __shared__ float4 s_h[NC * 8 * 64];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t o = __builtin_amdgcn_readfirstlane(blockIdx.x * DN_WAVES + tid / 64u);  // < H (H % 8 == 0)
+  const uint32_t cpr = I / 32u, nch = k * cpr;  // chunks of an expert's row, of an output row
+  float4 hv[NC];
 #pragma unroll
-      for (uint32_t u = 0; u < 8; ++u) {
-        const uint32_t i = base + u * blockDim.x;
-        if (i < n4) v[u] = h4[i];
-      }
+  for (int i = 0; i < NC; ++i)
+    hv[i] = reinterpret_cast<const float4*>(h)[min(tid + 512u * i, nch * 8u - 1u)];
+  uint32_t eo[NC];
+  float wr[NC];
+  bool ok[NC];
 #pragma unroll
-      for (uint32_t u = 0; u < 8; ++u) {
-        const uint32_t i = base + u * blockDim.x;
-        if (i < n4) s4[i] = v[u];
-      }
-    }
+  for (int i = 0; i < NC; ++i) {
+    const uint32_t c = lane + 64u * i, r = min(c, nch - 1u) / cpr;
+    const int32_t e = ids[r];
+    ok[i] = c < nch && static_cast<uint32_t>(e) < n_exp;
+    eo[i] = ok[i] ? static_cast<uint32_t>(e) : 0u;  // an absent chunk reads expert 0's row, its sum unused
+    wr[i] = wts[r];
+  }
+  uint4 q[NC];
+  uint16_t sc[NC], bi[NC];
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    const uint32_t col = min(lane + 64u * i, nch - 1u) % cpr;  // chunk within the expert's row
+    const uint64_t wrow = static_cast<uint64_t>(eo[i]) * H + o;
+    q[i] = load_stream(dw + wrow * (I / 8u) + 4u * col);
+    const uint64_t srow = wrow * (I / group) + 32u * col / group;
+    sc[i] = ds[srow];
+    bi[i] = db[srow];
+  }
+  __builtin_amdgcn_sched_barrier(0);  // the weights are on their way before h is waited for
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    const uint32_t f = tid + 512u * i, c = f / 8u, j = f % 8u;  // float4 j of chunk c
+    s_h[(c / 64u * 8u + j) * 64u + ((c % 64u) ^ j)] = hv[i];    // (past nch: a copy of the last, never used)
   }
   __syncthreads();
-  const uint32_t lane = threadIdx.x & 63;
-  const uint32_t r = lane >> 3, m = lane & 7;
-  const bool active_rank = r < k;
-  int32_t e = active_rank ? ids[r] : -1;
-  if (e >= static_cast<int32_t>(n_exp)) e = -1;
-  const float wr = (active_rank && e >= 0) ? wts[r] : 0.0f;
-  // this lane's h slice and per-block sums
-  float hf[CPL];
-  float hsum[BLK];
+  float acc = 0.0f;
 #pragma unroll
-  for (int c = 0; c < CPL; ++c) hf[c] = (active_rank && e >= 0) ? sh_h[r * I + m * CPL + c] : 0.0f;
+  for (int i = 0; i < NC; ++i) {
+    float hf[32], hs = 0.0f;
 #pragma unroll
-  for (int bl = 0; bl < BLK; ++bl) {
-    float s = 0.0f;
-#pragma unroll
-    for (int c = 0; c < 32; ++c) s = s + hf[bl * 32 + c];
-    hsum[bl] = s;
-  }
-  const uint32_t words = I / 8, groups = I / group;
-  const uint32_t wave = blockIdx.x * DN_WAVES + threadIdx.x / 64;
-#pragma unroll
-  for (int rr = 0; rr < DN_ROWS_PER_WAVE; ++rr) {
-    const uint32_t o = wave * DN_ROWS_PER_WAVE + rr;
-    if (o >= H) break;
-    float part = 0.0f;
-    if (e >= 0) {
-      const uint64_t wrow = static_cast<uint64_t>(e) * H + o;
-      const uint32_t* wp = dw + wrow * words + m * (CPL / 8);
-      const uint16_t* sp = ds + wrow * groups;
-      const uint16_t* bp = db + wrow * groups;
-#pragma unroll
-      for (int bl = 0; bl < BLK; ++bl) {
-        const uint4 q = *reinterpret_cast<const uint4*>(wp + 4 * bl);
-        const uint32_t gi = (m * CPL + 32 * bl) / group;
-        float a = 0.0f;
-        a = dot8_q4(q.x, hf + 32 * bl + 0, a);
-        a = dot8_q4(q.y, hf + 32 * bl + 8, a);
-        a = dot8_q4(q.z, hf + 32 * bl + 16, a);
-        a = dot8_q4(q.w, hf + 32 * bl + 24, a);
-        part = part + __builtin_fmaf(bf16_to_f32(sp[gi]), a, bf16_to_f32(bp[gi]) * hsum[bl]);
-      }
+    for (uint32_t j = 0; j < 8; ++j) {
+      const float4 v = s_h[(i * 8u + j) * 64u + (lane ^ j)];
+      hf[4 * j] = v.x; hf[4 * j + 1] = v.y; hf[4 * j + 2] = v.z; hf[4 * j + 3] = v.w;
+      hs = hs + ((v.x + v.y) + (v.z + v.w));
     }
-    // reduce the 8 lanes of each rank
-    part = part + __shfl_xor(part, 4, 64);
-    part = part + __shfl_xor(part, 2, 64);
-    part = part + __shfl_xor(part, 1, 64);
-    // combine in rank order
-    float acc = residual ? bf16_to_f32(residual[o]) : 0.0f;
-    for (uint32_t rk = 0; rk < k; ++rk) {
-      const float yr = __shfl(part, static_cast<int>(rk * 8), 64);
-      const float wk = __shfl(wr, static_cast<int>(rk * 8), 64);
-      acc = __builtin_fmaf(wk, yr, acc);
-    }
-    if (lane == 0) y[o] = f32_to_bf16(acc);
+    DotMix a{0.0f, 0.0f};
+    dot8_q4_mix(q[i].x, hf, a);
+    dot8_q4_mix(q[i].y, hf + 8, a);
+    dot8_q4_mix(q[i].z, hf + 16, a);
+    dot8_q4_mix(q[i].w, hf + 24, a);
+    const float part = __builtin_fmaf(bf16_to_f32(sc[i]), dot_mix_sum(a), bf16_to_f32(bi[i]) * hs);
+    acc = ok[i] ? __builtin_fmaf(wr[i], part, acc) : acc;
   }
+  acc = wave_sum_asc(acc);
+  if (lane == 0) y[o] = f32_to_bf16(residual ? bf16_to_f32(residual[o]) + acc : acc);
 }
 
 constexpr size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
@@ -228,38 +293,53 @@ int check_moe_layer(obs_ctx* ctx, const char* who, const obs_moe_layer* L) {
   return OBS_OK;
 }
 
+// norm_w (with eps): x is the layer's input and is normalised by the gate/up
+// launch; nullptr: x as it is.
 int launch_decode_experts(obs_ctx* ctx, const obs_moe_config* cfg, const obs_moe_layer* L, const uint16_t* x,
-                          const uint16_t* residual, uint16_t* y, const int32_t* ids, const float* w, float* h) {
+                          const uint16_t* norm_w, const uint16_t* residual, uint16_t* y, const int32_t* ids,
+                          const float* w, float* h) {
   const uint32_t H = cfg->hidden, I = cfg->inter, k = cfg->top_k, E = cfg->n_exp, G = cfg->group;
   const uint32_t rows = k * I;
-  const uint32_t gu_blocks = (rows + GU_WAVES * GU_ROWS_PER_WAVE - 1) / (GU_WAVES * GU_ROWS_PER_WAVE);
+#define OBS_GATEUP(W, CH, PR, NORM)                                                                               \
+  OBS_LAUNCH(ctx, "decode_gateup",                                                                                \
+             (decode_gateup_kernel<W, CH, PR, NORM>                                                               \
+              <<<(rows + GU_WAVES * PR - 1) / (GU_WAVES * PR), GU_WAVES * 64, 0, ctx->stream>>>(                  \
+                  L->gate_w, L->gate_s, L->gate_b, L->up_w, L->up_s, L->up_b, x, norm_w, cfg->rms_eps, ids, h, E, \
+                  k, I)))
+  // Row pairs per wave: as many as keep the launch at 8 waves per CU, at most 6
+  // (the registers of the rows in flight at H = 4096).
+#define OBS_GATEUP_ROWS(W, CH, NORM)                                      \
+  do {                                                                  \
+    if (rows <= GU_WAVES_MAX) OBS_GATEUP(W, CH, 1, NORM);                 \
+    else if (rows <= 2 * GU_WAVES_MAX) OBS_GATEUP(W, CH, 2, NORM);        \
+    else if (rows <= 4 * GU_WAVES_MAX) OBS_GATEUP(W, CH, 4, NORM);        \
+    else OBS_GATEUP(W, CH, 6, NORM);                                      \
+  } while (0)
+#define OBS_GATEUP_NORM(W, CH)                                            \
+  do {                                                                  \
+    if (norm_w) OBS_GATEUP_ROWS(W, CH, true);                             \
+    else OBS_GATEUP_ROWS(W, CH, false);                                   \
+  } while (0)
   switch (H) {
-    case 1024:
-      OBS_LAUNCH(ctx, "decode_gateup", decode_gateup_kernel<2><<<gu_blocks, GU_WAVES * 64, 0, ctx->stream>>>(L->gate_w, L->gate_s, L->gate_b, L->up_w, L->up_s, L->up_b, x, ids, h, E, k, H, I, G));
-      break;
-    case 2048:
-      OBS_LAUNCH(ctx, "decode_gateup", decode_gateup_kernel<4><<<gu_blocks, GU_WAVES * 64, 0, ctx->stream>>>(L->gate_w, L->gate_s, L->gate_b, L->up_w, L->up_s, L->up_b, x, ids, h, E, k, H, I, G));
-      break;
-    default:
-      OBS_LAUNCH(ctx, "decode_gateup", decode_gateup_kernel<8><<<gu_blocks, GU_WAVES * 64, 0, ctx->stream>>>(L->gate_w, L->gate_s, L->gate_b, L->up_w, L->up_s, L->up_b, x, ids, h, E, k, H, I, G));
-      break;
+    case 1024: OBS_GATEUP_NORM(2, 1); break;
+    case 2048: OBS_GATEUP_NORM(4, 1); break;
+    default: OBS_GATEUP_NORM(4, 2); break;
   }
-  const uint32_t dn_blocks = (H + DN_WAVES * DN_ROWS_PER_WAVE - 1) / (DN_WAVES * DN_ROWS_PER_WAVE);
-  const size_t lds = sizeof(float) * k * I;
-#define OBS_DOWN(CPL)                                                                                       \
-  OBS_LAUNCH(ctx, "decode_down",                                                                            \
-             decode_down_kernel<CPL><<<dn_blocks, DN_WAVES * 64, lds, ctx->stream>>>(L->down_w, L->down_s,  \
-                                                                                     L->down_b, h, ids, w,  \
-                                                                                     residual, y, E, k, H, I, G))
-  switch (I / 8) {
-    case 32: OBS_DOWN(32); break;
-    case 64: OBS_DOWN(64); break;
-    case 96: OBS_DOWN(96); break;
-    case 128: OBS_DOWN(128); break;
-    case 160: OBS_DOWN(160); break;
-    case 192: OBS_DOWN(192); break;
-    case 224: OBS_DOWN(224); break;
-    default: OBS_DOWN(256); break;
+#undef OBS_GATEUP_NORM
+#undef OBS_GATEUP_ROWS
+#undef OBS_GATEUP
+#define OBS_DOWN(NC)                                                                                              \
+  OBS_LAUNCH(ctx, "decode_down", (decode_down_kernel<NC><<<H / DN_WAVES, DN_WAVES * 64, 0, ctx->stream>>>(        \
+                                     L->down_w, L->down_s, L->down_b, h, ids, w, residual, y, E, k, H, I, G)))
+  switch ((rows / 32 + 63) / 64) {  // whole-wave loads per output row, at most 8
+    case 1: OBS_DOWN(1); break;
+    case 2: OBS_DOWN(2); break;
+    case 3: OBS_DOWN(3); break;
+    case 4: OBS_DOWN(4); break;
+    case 5: OBS_DOWN(5); break;
+    case 6: OBS_DOWN(6); break;
+    case 7: OBS_DOWN(7); break;
+    default: OBS_DOWN(8); break;
   }
 #undef OBS_DOWN
   return OBS_OK;
@@ -311,16 +391,21 @@ int decode_multi(obs_ctx* ctx, const obs_moe_config* cfg, const obs_moe_layer* l
   float* w = w_out ? w_out : reinterpret_cast<float*>(base + off_w);
   float* h = reinterpret_cast<float*>(base + off_h);
   int rc;
-  if (layer->norm_w) {  // the router and experts see rmsnorm(x) (forward.rs:419-421)
+  // The router and experts see rmsnorm(x) (forward.rs:419-421): normalised inside
+  // the router's and the gate/up launch, or by a launch of its own where the
+  // router takes two.
+  const uint16_t* norm_w = layer->norm_w;
+  if (norm_w && !route_one_launch(ctx, 1)) {
     uint16_t* xn = reinterpret_cast<uint16_t*>(base + off_xn);
-    rc = launch_rmsnorm(ctx, x, layer->norm_w, xn, 1, H, cfg->rms_eps);
+    rc = launch_rmsnorm(ctx, x, norm_w, xn, 1, H, cfg->rms_eps);
     if (rc) return rc;
     x = xn;
+    norm_w = nullptr;
   }
   rc = launch_route(ctx, layer->router_w, layer->router_s, layer->router_b, x, logits, ids, w, 1, H, E, cfg->group, k,
-                    cfg->norm_topk, cfg->route_rule);
+                    cfg->norm_topk, cfg->route_rule, norm_w, cfg->rms_eps);
   if (rc) return rc;
-  return launch_decode_experts(ctx, cfg, layer, x, residual, y, ids, w, h);
+  return launch_decode_experts(ctx, cfg, layer, x, norm_w, residual, y, ids, w, h);
 }
 
 }  // namespace obs

@@ -184,6 +184,14 @@ int launch_q4_rows_gemm(obs_ctx* ctx, RowsGemm which, const uint32_t* w, const u
 int launch_rmsnorm(obs_ctx* ctx, const uint16_t* x, const uint16_t* w, uint16_t* out, uint32_t rows, uint32_t dim,
                    float eps);
 
+// The router step (obs_router.hip): logits, then routing. norm_w (with eps):
+// the rows are normalised first, as launch_rmsnorm does; only where
+// route_one_launch() says that the step is one launch (nullptr elsewhere).
+bool route_one_launch(const obs_ctx* ctx, uint32_t T);
+int launch_route(obs_ctx* ctx, const uint32_t* w8, const uint16_t* s, const uint16_t* b, const uint16_t* x,
+                 float* logits, int32_t* ids, float* w, uint32_t T, uint32_t in, uint32_t n_exp, uint32_t group,
+                 uint32_t k, int norm_topk, int rule, const uint16_t* norm_w, float eps);
+
 // Fused single-launch decode (obs_decode_fused.hip).
 bool fused_decode_supported(const obs_moe_config* cfg);
 uint32_t fused_decode_workgroups();  // workgroups of one launch (each needs a CU of its own)

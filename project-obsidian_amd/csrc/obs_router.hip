@@ -45,13 +45,16 @@ constexpr int ROUTER_TOKENS_PER_WAVE = 8;
 // reads, ~20 dependent instructions) had cost as much as the pair's fmas.
 // The routing step of the one-launch router (obs_route): where the range's
 // ids and weights go, and the per-range counters that elect the workgroup
-// that routes (context memory, zero between launches).
+// that routes (context memory, zero between launches); with NORM the RMSNorm
+// weight and epsilon of the input rows.
 struct RouteTail {
   uint32_t* cnt;
   int32_t* ids;
   float* weights;
   uint32_t k;
   int norm_topk, rule;
+  const uint16_t* norm_w;
+  float eps;
 };
 
 // FUSED: the one-launch router for one token range (T <= 8). The grid is 8
@@ -62,7 +65,9 @@ struct RouteTail {
 // workgroup counts itself in cnt[0] once its logits are stored, and the last
 // to do so resets the counter and routes the range's tokens (route_topk_
 // kernel's per-token wave). NQ: logit slots per lane when routing.
-template <int WPL, int EPW, bool FUSED, int NQ>
+// NORM (with FUSED): each workgroup normalises the rows as it stages them, in
+// obs_rmsnorm's sequence, so a decode layer needs no launch for the norm.
+template <int WPL, int EPW, bool FUSED, int NQ, bool NORM = false>
 __global__ void __launch_bounds__(256) q8_gate_logits_kernel(const uint32_t* __restrict__ w8,
                                                              const uint16_t* __restrict__ s,
                                                              const uint16_t* __restrict__ b,
@@ -105,7 +110,36 @@ __global__ void __launch_bounds__(256) q8_gate_logits_kernel(const uint32_t* __r
     if (t0 >= T) break;  // uniform per workgroup
     const uint32_t nt = min(static_cast<uint32_t>(ROUTER_TOKENS_PER_WAVE), T - t0);
     if (ci > 0) __syncthreads();  // the previous chunk's activations and partials are read
-    {
+    if constexpr (NORM) {
+      for (uint32_t t = wave; t < nt; t += 4u) {  // one wave per row, the lane's C columns
+        uint4 xv[C / 8], nv[C / 8];
+#pragma unroll
+        for (int i = 0; i < C / 8; ++i) {
+          xv[i] = reinterpret_cast<const uint4*>(x + static_cast<uint64_t>(t) * in + lane * C)[i];
+          nv[i] = reinterpret_cast<const uint4*>(rt.norm_w + lane * C)[i];
+        }
+        float ss = 0.0f;
+#pragma unroll
+        for (int i = 0; i < C / 8; ++i) {
+          const uint32_t d[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w};
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            ss = __builtin_fmaf(bf16lo(d[j]), bf16lo(d[j]), ss);
+            ss = __builtin_fmaf(bf16hi(d[j]), bf16hi(d[j]), ss);
+          }
+        }
+        const float inv = 1.0f / __builtin_sqrtf(wave_sum_asc(ss) / static_cast<float>(in) + rt.eps);
+#pragma unroll
+        for (int i = 0; i < C / 8; ++i) {
+          const uint32_t d[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w}, g[4] = {nv[i].x, nv[i].y, nv[i].z, nv[i].w};
+          uint32_t o[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            o[j] = pack_bf16x2((bf16lo(d[j]) * inv) * bf16lo(g[j]), (bf16hi(d[j]) * inv) * bf16hi(g[j]));
+          *reinterpret_cast<uint4*>(s_x + t * in + lane * C + 8 * i) = make_uint4(o[0], o[1], o[2], o[3]);
+        }
+      }
+    } else {
       // (the next chunk's rows loaded into registers during this chunk measured
       // slower: 41 against 33 us per layer at 2,048 tokens)
       const uint32_t row_chunks = in / 8u;  // 16-byte chunks per activation row
@@ -287,9 +321,11 @@ int launch_route_fused(obs_ctx* ctx, const uint32_t* w8, const uint16_t* s, cons
                        float* logits, uint32_t T, uint32_t in, uint32_t n_exp, uint32_t group, const RouteTail& rt) {
   const dim3 grid(8u * ((n_exp + 3) / 4), 1);
   const size_t lds = sizeof(uint16_t) * ROUTER_TOKENS_PER_WAVE * in;
-#define OBS_ROUTE1(WPL)                                                                                 \
-  OBS_LAUNCH(ctx, "route_fused", (q8_gate_logits_kernel<WPL, 1, true, NQ><<<grid, 256, lds, ctx->stream>>>( \
+#define OBS_ROUTE2(WPL, NORM)                                                                                     \
+  OBS_LAUNCH(ctx, "route_fused", (q8_gate_logits_kernel<WPL, 1, true, NQ, NORM><<<grid, 256, lds, ctx->stream>>>( \
                                      w8, s, b, x, logits, T, in, n_exp, group, 1u, rt)))
+#define OBS_ROUTE1(WPL) \
+  if (rt.norm_w) OBS_ROUTE2(WPL, true); else OBS_ROUTE2(WPL, false)
   switch (in) {
     case 512: OBS_ROUTE1(2); break;
     case 1024: OBS_ROUTE1(4); break;
@@ -297,14 +333,19 @@ int launch_route_fused(obs_ctx* ctx, const uint32_t* w8, const uint16_t* s, cons
     default: OBS_ROUTE1(16); break;
   }
 #undef OBS_ROUTE1
+#undef OBS_ROUTE2
   return OBS_OK;
+}
+
+bool route_one_launch(const obs_ctx* ctx, uint32_t T) {
+  return T <= static_cast<uint32_t>(ROUTER_TOKENS_PER_WAVE) && ctx->xcd_map_ok;
 }
 
 int launch_route(obs_ctx* ctx, const uint32_t* w8, const uint16_t* s, const uint16_t* b, const uint16_t* x,
                  float* logits, int32_t* ids, float* w, uint32_t T, uint32_t in, uint32_t n_exp, uint32_t group,
-                 uint32_t k, int norm_topk, int rule) {
-  if (T <= static_cast<uint32_t>(ROUTER_TOKENS_PER_WAVE) && ctx->xcd_map_ok) {
-    const RouteTail rt{ctx->route_cnt, ids, w, k, norm_topk, rule};
+                 uint32_t k, int norm_topk, int rule, const uint16_t* norm_w, float eps) {
+  if (route_one_launch(ctx, T)) {
+    const RouteTail rt{ctx->route_cnt, ids, w, k, norm_topk, rule, norm_w, eps};
     if (n_exp <= 64) return launch_route_fused<1>(ctx, w8, s, b, x, logits, T, in, n_exp, group, rt);
     if (n_exp <= 128) return launch_route_fused<2>(ctx, w8, s, b, x, logits, T, in, n_exp, group, rt);
     return launch_route_fused<4>(ctx, w8, s, b, x, logits, T, in, n_exp, group, rt);
@@ -347,7 +388,8 @@ int obs_route(obs_ctx* ctx, const uint32_t* w8, const uint16_t* scales, const ui
   if (!obs::aligned(x, 16) || !obs::aligned(w8, 16))
     return obs::set_error(ctx, OBS_E_ALIGN, "obs_route: x and w8 must be 16-byte aligned");
   if (T == 0) return OBS_OK;
-  return obs::launch_route(ctx, w8, scales, biases, x, logits, ids, weights, T, in, n_exp, group, k, norm_topk, rule);
+  return obs::launch_route(ctx, w8, scales, biases, x, logits, ids, weights, T, in, n_exp, group, k, norm_topk, rule,
+                           nullptr, 0.0f);
 }
 
 int obs_route_topk(obs_ctx* ctx, const float* logits, int32_t* ids, float* weights, uint32_t T,

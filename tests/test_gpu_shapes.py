@@ -92,6 +92,40 @@ def test_decode_widest_shape(exe):
     _close(_f32(y), y64[0], 1e-2)
 
 
+# The multi-launch decode's row splits: gate/up rows per wave 1, 2, 4 and 6 (with a
+# last wave of fewer rows), 1 to 8 whole-wave loads per down row (the last one
+# partly filled), every width.
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("E,H,I,K", [(8, 1024, 256, 1), (8, 4096, 256, 3), (8, 1024, 512, 8), (9, 2048, 768, 7),
+                                     (8, 4096, 1536, 5), (8, 2048, 1280, 7), (8, 4096, 1792, 6), (8, 1024, 2048, 7),
+                                     (16, 4096, 2048, 8), (8, 2048, 2048, 8)])
+def test_decode_multi_row_splits(exe, E, H, I, K, norm):
+    """Every output is one rounding to bf16 (half a unit of 8 bits, 2^-8 relative) of fp32 sums (some 1e-6)."""
+    t = synth.moe_layer(50 + H + I + K, E, H, I, 64)
+    rng = np.random.default_rng(H + I + K)
+    x, res = synth.bf16_normal(rng, H), synth.bf16_normal(rng, H)
+    xn, table = x, t
+    if norm:
+        nw = synth.bf16_normal(rng, H)
+        table, xn = dict(t, norm_w=nw), O.rmsnorm(x, nw, 1e-6)
+    layer = oh.MoeLayer.upload(exe, table)
+    L = O.Layer(t, E, H, I, 64)
+    cfg = oh.MoeConfig(E, K, H, I, 64, True, rms_eps=1e-6)
+    exe.set_decode_path(oh.OBS_DECODE_MULTI)
+    try:
+        y, ids, w = exe.alloc(H, np.uint16), exe.alloc(K, np.int32), exe.alloc(K, np.float32)
+        exe.moe_decode(cfg, layer, exe.upload(x), y, residual=exe.upload(res), ids_out=ids, w_out=w)
+    finally:
+        exe.set_decode_path(oh.OBS_DECODE_AUTO)
+    _, ri, rw = O.router(L, xn, K, True)
+    assert np.array_equal(ids.download(), ri[0])
+    assert np.array_equal(w.download().view(np.uint32), rw[0].view(np.uint32))
+    y64, _, _ = O.moe_decode(L, xn, K, True, ids=ri, w=rw)
+    ref = y64[0] + _f32(res)
+    got = _f32(y.download())
+    assert np.all(np.abs(got - ref) <= 2.0 ** -8 * np.abs(ref) + 1e-5 * np.sqrt(np.mean(ref ** 2)))
+
+
 @pytest.mark.parametrize("E,H,I,K,T", [(256, 2048, 768, 8, 96), (64, 2048, 768, 8, 130), (32, 1024, 512, 4, 77)])
 def test_prefill_shapes(exe, E, H, I, K, T):
     t = synth.moe_layer(40 + E + H, E, H, I, 64)
