@@ -110,6 +110,26 @@ def test_q8_gate_logits_other_widths_bit_exact(exe, H, E, T):
         assert np.array_equal(got[t].view(np.uint32), ref.view(np.uint32)), f"token {t}"
 
 
+# The matrix-core logits (from 65 tokens): each width, the last tile of tokens and of
+# experts partly filled, groups shorter than a lane's columns, several tiles per
+# workgroup (over 1,024 tokens at 128 experts, 512 at 256).
+@pytest.mark.parametrize("H,E,T,group", [(512, 60, 65, 64), (512, 16, 129, 4), (1024, 128, 80, 8), (2048, 17, 97, 16),
+                                         (2048, 256, 700, 64), (4096, 33, 130, 32), (4096, 128, 600, 64)])
+def test_q8_gate_logits_tiles_bit_exact(exe, H, E, T, group):
+    """Bit for bit the reduction order, also where sums go through subnormals."""
+    rng = np.random.default_rng(320 + H + E + T)
+    w, s, b = synth.quant_tensor(rng, E, H, 8, group)
+    x = synth.bf16_normal(rng, (T, H))
+    x[T // 2] = synth.bf16_normal(rng, H, 2.0 ** -126)
+    lg = exe.alloc((T, E), np.float32)
+    exe.q8_gate_logits(exe.upload(w), exe.upload(s), exe.upload(b), exe.upload(x), lg, T, H, E, group)
+    got = lg.download()
+    xf = _f32(x)
+    for t in sorted({0, 15, 16, T // 2, T - 2, T - 1, *rng.integers(0, T, 20)}):
+        ref = O.qmatvec("lanes", 8, w, s, b, xf[t], H, E, lanes=64, group=group)
+        assert np.array_equal(got[t].view(np.uint32), ref.view(np.uint32)), f"token {t}"
+
+
 @pytest.mark.parametrize("rule", [O.ROUTE_REF, O.ROUTE_F32], ids=["ref", "f32"])
 @pytest.mark.parametrize("n_exp,k,norm", [(128, 8, True), (128, 8, False), (64, 4, True), (256, 8, True),
                                           (100, 7, True), (16, 16, True), (128, 1, True)])
