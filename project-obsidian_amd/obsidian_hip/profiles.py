@@ -40,9 +40,7 @@ KERNELS = {
     "grouped_gemm_gateup": (r"grouped_gemm_kernel<1u, 3u>", ("csrc/obs_prefill.hip", "csrc/obs_internal.hpp")),
     "grouped_gemm_down": (r"grouped_gemm_kernel<2u, 5u>", ("csrc/obs_prefill.hip", "csrc/obs_internal.hpp")),
     "moe_ffn": (r"moe_ffn_kernel<2u>", ("csrc/obs_prefill.hip", "csrc/obs_internal.hpp")),
-    "moe_group_count": (r"group_count_kernel", ("csrc/obs_prefill.hip",)),
-    "moe_group_scan": (r"group_scan_kernel", ("csrc/obs_prefill.hip",)),
-    "moe_group_rank": (r"group_rank_kernel", ("csrc/obs_prefill.hip",)),
+    "moe_group": (r"group_kernel<", ("csrc/obs_prefill.hip",)),
     "moe_combine": (r"combine_kernel", ("csrc/obs_prefill.hip",)),
 }
 COPY = r"copyBuffer"

@@ -351,6 +351,38 @@ def test_moe_prefill_invalid_and_duplicate_ids_are_skipped(exe, qwen):
     _close(y, ref, BF_NORM, BF_ELEM)
 
 
+@pytest.mark.parametrize("T,k,offset", [(1, 8, 0), (64, 8, 4), (256, 8, 0), (257, 8, 0), (257, 8, 4), (1025, 8, 0),
+                                        (1025, 6, 0), (1100, 1, 0)])
+def test_moe_prefill_grouping_forms(exe, T, k, offset):
+    """The grouping reads eight aligned ids of a token at once, else one by one,
+    with 4 or 16 waves an expert: both forms over tokens that fill their waves'
+    ranges or not, with ids skipped (out of range, repeated) at their edges."""
+    e, h, i = 16, 1024, 256
+    t = synth.moe_layer(33, e, h, i, 64)
+    layer, L = oh.MoeLayer.upload(exe, t), O.Layer(t, e, h, i, 64)
+    cfg = oh.MoeConfig(e, k, h, i, 64, True)
+    rng = np.random.default_rng(991 + T + k)
+    X = synth.bf16_normal(rng, (T, h))
+    ids, w = synth.zipf_routing(T, e, k, 1.1, seed=13)
+    bad, wz = ids.copy(), w.copy()
+    for tt in {0, T // 2, T - 1}:
+        bad[tt, k - 1] = bad[tt, 0] if k > 1 else -1  # a repeat of an earlier rank
+        wz[tt, k - 1] = 0.0
+        if k > 2:
+            bad[tt, 1] = e  # out of range
+            wz[tt, 1] = 0.0
+    raw = exe.alloc(offset + bad.nbytes, np.uint8)
+    raw.upload(np.concatenate([np.zeros(offset, np.uint8), np.ascontiguousarray(bad, np.int32).view(np.uint8).ravel()]))
+    ws, Y = exe.alloc(exe.moe_prefill_workspace(cfg, T), np.uint8), exe.alloc((T, h), np.uint16)
+    exe.moe_prefill(cfg, layer, exe.upload(X), Y, T, ids=raw.ptr + offset, weights=exe.upload(w.astype(np.float32)),
+                    ws=ws, ws_bytes=ws.nbytes)
+    exe.device_status()
+    y = _f32(Y.download())
+    assert np.all(np.isfinite(y))
+    sel = np.unique(np.concatenate([[0, T // 2, T - 1], rng.integers(0, T, 60)]))
+    _close(y[sel], O.moe_prefill(L, X[sel], ids[sel], wz[sel], O.MODE_MFMA_BF16), BF_NORM, BF_ELEM)
+
+
 def test_moe_prefill_workspace_and_shape_errors(exe, qwen):
     _, layer, _ = qwen
     cfg = oh.MoeConfig(E, K, H, I, 64, True)
