@@ -133,7 +133,11 @@ def test_q4_matmul_weight_operand_bit_exact(exe, huge):
 # does not take.
 @pytest.mark.parametrize("T,in_f,out_f", [(1, 256, 128), (31, 2048, 128), (33, 768, 256), (32, 4096, 128),
                                           (37, 2048, 5120), (65, 2304, 5120), (129, 2048, 5120), (333, 512, 5120),
-                                          (300, 768, 5120), (1000, 4096, 2048)])
+                                          (300, 768, 5120), (1000, 4096, 2048),
+                                          # 96 x 128, 128 x 128, 96 x 256, 128 x 256, 160 x 256 tiles (ragged, full)
+                                          (481, 2048, 5120), (480, 2048, 5120), (701, 2048, 5120), (640, 2048, 5120),
+                                          (1001, 2048, 5120), (960, 512, 5120), (1290, 2048, 5120), (1889, 2048, 5120),
+                                          (1920, 2048, 5120), (1889, 4096, 2048), (2500, 4096, 2048)])
 def test_q4_matmul_few_rows(exe, T, in_f, out_f):
     """5e-3 against the kernel's bf16 operands in fp64: the fp32 sums differ by
     1e-6, the bf16 output by half a step (2^-9)."""
@@ -150,7 +154,11 @@ def test_q4_matmul_few_rows(exe, T, in_f, out_f):
 
 
 @pytest.mark.parametrize("T,in_f,out_f,huge", [(64, 2048, 5120, False), (64, 2048, 5120, True),
-                                               (200, 2048, 5120, False), (200, 2048, 5120, True)])
+                                               (200, 2048, 5120, False), (200, 2048, 5120, True),
+                                               (481, 2048, 5120, True), (701, 2048, 5120, True),
+                                               (1001, 2048, 5120, False), (1001, 2048, 5120, True),
+                                               (1290, 2048, 5120, True), (1889, 2048, 5120, False),
+                                               (1889, 2048, 5120, True)])
 def test_q4_matmul_few_rows_operand_bit_exact(exe, T, in_f, out_f, huge):
     """As test_q4_matmul_weight_operand_bit_exact (which takes the 32-row
     kernel), for the 64-row and the K-in-two kernels: row t is one-hot at column
