@@ -66,6 +66,31 @@ def test_attn_prep_rows_vs_oracle(exe, pos0, T):
     assert np.array_equal(gk[:, keep], kc0[:, keep]) and np.array_equal(gv[:, :, keep], vc0[:, :, keep])
 
 
+@pytest.mark.parametrize("nh,nkv,T", [(32, 4, 1), (32, 4, 67), (16, 4, 5), (6, 3, 9), (1, 1, 2)])
+def test_attn_prep_rows_forms_agree(exe, nh, nkv, T):
+    """At 16-byte alignment four heads share a wave; at 4-byte alignment a head
+    has its own. Same sums in the same order: bit for bit, q/k/v as column
+    ranges of one buffer, head counts that do not fill a wave among them."""
+    hd, ml, pos0 = 128, 96, 11
+    ld = (nh + 2 * nkv) * hd
+    rng = np.random.default_rng(1250 + T + nh)
+    rows = synth.bf16_normal(rng, (T, ld), 2.0)
+    norms = [exe.upload(synth.bf16_normal(rng, hd, 0.5)) for _ in range(2)]
+    got = []
+    for off in (0, 2):  # elements
+        buf = exe.upload(np.concatenate([np.zeros(off, np.uint16), rows.reshape(-1)]))
+        q = buf.ptr + 2 * off
+        kc, vc = exe.alloc((nkv, ml, hd), np.uint16), exe.alloc((nkv, hd, ml), np.uint16)
+        for c in (kc, vc):
+            c.upload(np.full(c.shape, 0x1234, np.uint16))
+        exe.attn_prep_rows(q, q + 2 * nh * hd, q + 2 * (nh + nkv) * hd, norms[0], norms[1], kc, vc, nh, nkv, hd, ml,
+                           EPS, THETA, pos0, T, q_ld=ld, kv_ld=ld)
+        got.append((buf.download()[off:], kc.download(), vc.download()))
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+    assert not np.array_equal(got[0][0], rows.reshape(-1))
+
+
 @pytest.mark.parametrize("nh,nkv,pos0,T", [(32, 4, 0, 1), (32, 4, 0, 9), (32, 4, 31, 2), (32, 4, 500, 37),
                                            (32, 4, 3990, 106), (16, 1, 7, 5), (16, 4, 60, 11)])
 def test_sdpa_prefill_vs_oracle(exe, nh, nkv, pos0, T):
