@@ -778,11 +778,21 @@ __global__ void __launch_bounds__(GROUP_TPB) group_kernel(const int32_t* __restr
 
 // y[t, :] = residual + sum_r w[t, r] * Yp[t*k + r, :] (fp32, rank order). One
 // workgroup per token (H / 8 threads, 8 columns each): the token's ids and
-// weights are uniform, so they load once into scalar registers.
+// weights are uniform, so they load once into scalar registers. All (up to 8)
+// rows are requested before the first is added: with few tokens the kernel is
+// bound by its latency, and a row under the branch that skips it waited for the
+// row before. Rows the grouping skipped (never written) are read, not added.
+// H 2,048, k 8: 37 tokens 6.8 -> 5.2 us, 333 8.2 -> 6.2, 2,048 16.2 -> 14.9 (84 MB,
+// 5.6 TB/s).
 __global__ void __launch_bounds__(512) combine_kernel(const uint16_t* __restrict__ Yp, const int32_t* __restrict__ ids,
                                                       const float* __restrict__ w, const uint16_t* __restrict__ residual,
                                                       uint16_t* __restrict__ y, uint32_t k, uint32_t H, uint32_t E) {
   const uint32_t t = blockIdx.x, c = 8u * threadIdx.x;
+  const size_t row0 = static_cast<size_t>(t) * k;
+  uint4 v[8];
+#pragma unroll
+  for (uint32_t r = 0; r < 8; ++r)  // ranks past k read the last one again, unused
+    v[r] = *reinterpret_cast<const uint4*>(Yp + (row0 + min(r, k - 1u)) * H + c);
   float acc[8];
   if (residual) {
     const uint4 rv = *reinterpret_cast<const uint4*>(residual + static_cast<size_t>(t) * H + c);
@@ -792,18 +802,25 @@ __global__ void __launch_bounds__(512) combine_kernel(const uint16_t* __restrict
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
   }
-  const int32_t* tid_ids = ids + static_cast<size_t>(t) * k;
-  for (uint32_t r = 0; r < k; ++r) {
-    const int32_t e = tid_ids[r];
-    bool skip = e < 0 || static_cast<uint32_t>(e) >= E;  // rows the grouping skipped
-    for (uint32_t q = 0; q < r; ++q) skip = skip || tid_ids[q] == e;
+  int32_t id[8];
+  float wr[8];
+#pragma unroll
+  for (uint32_t r = 0; r < 8; ++r) {
+    id[r] = ids[row0 + min(r, k - 1u)];
+    wr[r] = w[row0 + min(r, k - 1u)];
+  }
+#pragma unroll
+  for (uint32_t r = 0; r < 8; ++r) {
+    bool skip = r >= k || id[r] < 0 || static_cast<uint32_t>(id[r]) >= E;  // rows the grouping skipped
+#pragma unroll
+    for (uint32_t q = 0; q < r; ++q) skip = skip || id[q] == id[r];
     if (skip) continue;
-    const float wr = w[static_cast<size_t>(t) * k + r];
-    const uint4 v = *reinterpret_cast<const uint4*>(Yp + (static_cast<size_t>(t) * k + r) * H + c);
-    acc[0] = __builtin_fmaf(wr, bf16lo(v.x), acc[0]); acc[1] = __builtin_fmaf(wr, bf16hi(v.x), acc[1]);
-    acc[2] = __builtin_fmaf(wr, bf16lo(v.y), acc[2]); acc[3] = __builtin_fmaf(wr, bf16hi(v.y), acc[3]);
-    acc[4] = __builtin_fmaf(wr, bf16lo(v.z), acc[4]); acc[5] = __builtin_fmaf(wr, bf16hi(v.z), acc[5]);
-    acc[6] = __builtin_fmaf(wr, bf16lo(v.w), acc[6]); acc[7] = __builtin_fmaf(wr, bf16hi(v.w), acc[7]);
+    const uint32_t vw[4] = {v[r].x, v[r].y, v[r].z, v[r].w};
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+      acc[2 * j] = __builtin_fmaf(wr[r], bf16lo(vw[j]), acc[2 * j]);
+      acc[2 * j + 1] = __builtin_fmaf(wr[r], bf16hi(vw[j]), acc[2 * j + 1]);
+    }
   }
   *reinterpret_cast<uint4*>(y + static_cast<size_t>(t) * H + c) =
       make_uint4(pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3]), pack_bf16x2(acc[4], acc[5]),
