@@ -173,15 +173,6 @@ void* stream_scratch(obs_ctx* ctx, size_t bytes);
 // has nblk 32-position blocks, on a device with `cus` CUs (obs_attention.hip).
 uint32_t sdpa_prefill_splits(uint32_t wgs, uint32_t nblk, uint32_t cus);
 
-// Dense 4-bit GEMM of few rows (obs_rows_gemm.hip): which of its kernels a size
-// takes (NONE: the 128-row tiles of obs_prefill.hip; T*: tiles of that many rows
-// x 128 columns, W: 256), and the launch.
-enum class RowsGemm { NONE, R32, R64, KSPLIT, T96, T128, T96W, T128W, T160W };
-int rows_gemm_init(obs_ctx* ctx);
-RowsGemm q4_rows_gemm_pick(uint32_t T, uint32_t K, uint32_t N, uint32_t cus);
-int launch_q4_rows_gemm(obs_ctx* ctx, RowsGemm which, const uint32_t* w, const uint16_t* s, const uint16_t* b,
-                        const uint16_t* X, uint16_t* Y, uint32_t T, uint32_t K, uint32_t N);
-
 // RMSNorm of rows x dim bf16 (obs_elementwise.hip); dim % 64 == 0, <= 8192.
 int launch_rmsnorm(obs_ctx* ctx, const uint16_t* x, const uint16_t* w, uint16_t* out, uint32_t rows, uint32_t dim,
                    float eps);

@@ -126,15 +126,11 @@ def test_q4_matmul_weight_operand_bit_exact(exe, huge):
     assert np.array_equal(got, ref), int(np.sum(got != ref))
 
 
-# The K-splitting kernels of few rows at the edges of their tiles: 32-row tiles
-# (1, 31, 32, 33 rows; one to sixteen K units for 8 waves), 64-row tiles (from
-# 256 tiles of 32 rows on) and 64 x 128 tiles with K in two sets (from 256 tiles
-# of 64 x 32 on, K a multiple of 512), and T = 300 of K = 768, which that one
-# does not take.
+# Row counts around the 32-row blocks and the 128-row tiles, from one row to 20
+# tiles; K of 4 to 64 groups, N of one to 40 column blocks.
 @pytest.mark.parametrize("T,in_f,out_f", [(1, 256, 128), (31, 2048, 128), (33, 768, 256), (32, 4096, 128),
                                           (37, 2048, 5120), (65, 2304, 5120), (129, 2048, 5120), (333, 512, 5120),
                                           (300, 768, 5120), (1000, 4096, 2048),
-                                          # 96 x 128, 128 x 128, 96 x 256, 128 x 256, 160 x 256 tiles (ragged, full)
                                           (481, 2048, 5120), (480, 2048, 5120), (701, 2048, 5120), (640, 2048, 5120),
                                           (1001, 2048, 5120), (960, 512, 5120), (1290, 2048, 5120), (1889, 2048, 5120),
                                           (1920, 2048, 5120), (1889, 4096, 2048), (2500, 4096, 2048)])
@@ -160,9 +156,9 @@ def test_q4_matmul_few_rows(exe, T, in_f, out_f):
                                                (1290, 2048, 5120, True), (1889, 2048, 5120, False),
                                                (1889, 2048, 5120, True)])
 def test_q4_matmul_few_rows_operand_bit_exact(exe, T, in_f, out_f, huge):
-    """As test_q4_matmul_weight_operand_bit_exact (which takes the 32-row
-    kernel), for the 64-row and the K-in-two kernels: row t is one-hot at column
-    (37 t) % in_f, so Y[t] is that column of the bf16 weight operand."""
+    """As test_q4_matmul_weight_operand_bit_exact, at a projection's width and from
+    half a tile to 15: row t is one-hot at column (37 t) % in_f, so Y[t] is that
+    column of the bf16 weight operand."""
     rng = np.random.default_rng(4300 + T + huge)
     w = rng.integers(0, 2**32, size=(out_f, in_f // 8), dtype=np.uint64).astype(np.uint32)
     s, b = _extreme_scales(rng, out_f, in_f // 64, huge)
@@ -176,9 +172,28 @@ def test_q4_matmul_few_rows_operand_bit_exact(exe, T, in_f, out_f, huge):
     assert np.array_equal(got, ref), int(np.sum(got != ref))
 
 
+@pytest.mark.parametrize("in_f,out_f,Ts", [(2048, 5120, (1, 24, 37, 64, 200, 333, 500, 701, 1001, 1300, 1900)),
+                                           (4096, 2048, (24, 129, 512, 1300, 1900)), (768, 2048, (40, 300))])
+def test_q4_matmul_row_does_not_depend_on_the_batch(exe, in_f, out_f, Ts):
+    """A row's output is the same bits whatever rows are batched with it: its sum
+    over K runs in one order at every size. (Two orders differ by a rounding of the
+    bf16 output here and there, which a few layers on is another set of experts for
+    a token whose 8th and 9th router logits are close.)"""
+    rng = np.random.default_rng(4600 + in_f)
+    w, s, b = synth.centered_quant(rng, out_f, in_f)
+    big = 2048  # 256-column tiles at 5,120 columns
+    X = exe.upload(synth.bf16_normal(rng, (big, in_f)))
+    dw, ds, db, Y = exe.upload(w), exe.upload(s), exe.upload(b), exe.alloc((big, out_f), np.uint16)
+    exe.q4_matmul(dw, ds, db, X, Y, big, in_f, out_f, 64)
+    want = Y.download()
+    for T in Ts:
+        exe.q4_matmul(dw, ds, db, X, Y, T, in_f, out_f, 64)
+        got = Y.download()[:T]
+        assert np.array_equal(got, want[:T]), (T, int(np.sum(got != want[:T])))
+
+
 def test_q4_matmul_scales_at_two_byte_alignment(exe):
-    """Scales and biases that are not 8-byte aligned keep the 128-row tiles,
-    with the same result to the rounding of their sums' order."""
+    """Scales and biases need no alignment beyond their own 2 bytes."""
     T, in_f, out_f = 40, 2048, 768
     rng = np.random.default_rng(4400)
     w, s, b = synth.centered_quant(rng, out_f, in_f)
