@@ -462,7 +462,8 @@ int obs_attn_prep_rows(obs_ctx* ctx, uint16_t* q, const uint16_t* k, const uint1
 /* Causal GQA attention of a prefill batch (the per-token Attention::sdpa of
  * forward.rs:155 for tokens at positions pos0 + t): token t attends to cache
  * positions [0, pos0 + t]; the batch's keys and values must be in the caches
- * (obs_attn_prep_rows first). q bf16 rows of q_ld elements (a multiple of 8;
+ * (obs_attn_prep_rows first). A token's output is the same bits in any batch
+ * and in a replayed capture. q bf16 rows of q_ld elements (a multiple of 8;
  * 0 = dense) holding [n_heads, head_dim]; out bf16 [n_tokens, n_heads,
  * head_dim]; head_dim 128, query heads per kv head a divisor of 16; q, out
  * and both caches 16-byte aligned (OBS_E_ALIGN). */

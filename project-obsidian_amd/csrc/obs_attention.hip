@@ -650,24 +650,12 @@ constexpr uint32_t PF_BUF = 32u * PF_KROW + HD * PF_VROW;  // bf16 elements per 
 
 constexpr uint32_t PF_THREADS = 512;  // two sets of 4 waves
 
-// SPLIT: `splits` workgroups share a (tile, kv head), each running a contiguous
-// run of its blocks, and leave unnormalised partials for
-// sdpa_prefill_combine_kernel: per (tile, split, kv head) O [128 columns][128]
-// fp32, then m [128] and l [128] (column = token of the tile x G + head). The
-// kernel is a serial chain of blocks (~1.4 us per two), so few tokens over a
-// long cache left it to a handful of workgroups: 57 tokens at position 3,500
-// are 16 workgroups of 112 blocks.
-constexpr uint32_t PF_COLS = 128u;                            // columns of a tile
-constexpr uint32_t PF_PART = PF_COLS * HD + 2u * PF_COLS;      // floats of one partial
-
-template <bool SPLIT>
 __global__ void __launch_bounds__(PF_THREADS, 1) sdpa_prefill_kernel(const uint16_t* __restrict__ q,
                                                                     const uint16_t* __restrict__ k_cache,
                                                                     const uint16_t* __restrict__ v_cache_t,
                                                                     uint16_t* __restrict__ out, uint32_t nh,
                                                                     uint32_t nkv, uint32_t max_len, uint32_t pos0,
-                                                                    uint32_t n_tok, uint32_t q_ld, float scale_log2,
-                                                                    uint32_t splits, float* __restrict__ part) {
+                                                                    uint32_t n_tok, uint32_t q_ld, float scale_log2) {
   // per set, two staging buffers; after the block loop the second set's
   // (m, l, O) pass through them to the first
   __shared__ __attribute__((aligned(16))) uint16_t s_blk[2][2][PF_BUF];
@@ -678,15 +666,12 @@ __global__ void __launch_bounds__(PF_THREADS, 1) sdpa_prefill_kernel(const uint1
   // tiles in launch order from the longest (last tokens) down: one workgroup
   // fills a CU, so the dispatcher hands the shorter tiles to the CUs that free
   // up first
-  const uint32_t kv = blockIdx.x % nkv, rs = blockIdx.x / nkv;
-  const uint32_t r = SPLIT ? rs / splits : rs, sp = SPLIT ? rs % splits : 0u;
-  const uint32_t tile = n_wg_tok - 1u - r, tb = tile * TPWG;  // first token
+  const uint32_t kv = blockIdx.x % nkv, r = blockIdx.x / nkv;
+  const uint32_t tb = (n_wg_tok - 1u - r) * TPWG;  // first token
   const uint32_t col = lane & 15u, g = lane >> 4;
   const uint32_t cj = col / G, ci = col % G;
   const uint32_t seq = pos0 + min(tb + TPWG, n_tok);  // the workgroup's longest sequence
-  // the workgroup's blocks: [blk0, blk0 + nblk) (a split of a short tile may have none)
-  const uint32_t nall = (seq + 31u) / 32u, per = SPLIT ? (nall + splits - 1u) / splits : nall;
-  const uint32_t blk0 = min(sp * per, nall), nblk = min(per, nall - blk0);
+  const uint32_t nblk = (seq + 31u) / 32u;
   // the wave's two column groups: query slices (B operand), limits, state
   bf16x8_t qb[2][4];
   uint32_t lim[2];
@@ -863,10 +848,7 @@ __global__ void __launch_bounds__(PF_THREADS, 1) sdpa_prefill_kernel(const uint1
   // last block is loaded again (unused). Both sets run the same iterations, so
   // all 8 waves meet every barrier.
   const uint32_t nit = (nblk + 1u) / 2u;
-  // (clamped to the tile's last block where a split has none: loaded, not used)
-  auto blk_of = [&](uint32_t i) __attribute__((always_inline)) {
-    return SPLIT ? min(blk0 + min(2u * i + set, max(nblk, 1u) - 1u), nall - 1u) : min(2u * i + set, nblk - 1u);
-  };
+  auto blk_of = [&](uint32_t i) __attribute__((always_inline)) { return min(2u * i + set, nblk - 1u); };
   u32x4_t sa[4], sb[4];
   load_blk(blk_of(0u), sa);
   load_blk(blk_of(1u), sb);
@@ -874,12 +856,12 @@ __global__ void __launch_bounds__(PF_THREADS, 1) sdpa_prefill_kernel(const uint1
   __syncthreads();
   for (uint32_t i = 0;;) {
     load_blk(blk_of(i + 2u), sa);
-    if (2u * i + set < nblk) run_blk(0u, blk0 + 2u * i + set);  // uniform per set
+    if (2u * i + set < nblk) run_blk(0u, 2u * i + set);  // uniform per set
     store_blk(1u, sb, blk_of(i + 1u));
     __syncthreads();
     if (++i >= nit) break;
     load_blk(blk_of(i + 2u), sb);
-    if (2u * i + set < nblk) run_blk(1u, blk0 + 2u * i + set);
+    if (2u * i + set < nblk) run_blk(1u, 2u * i + set);
     store_blk(0u, sa, blk_of(i + 1u));
     __syncthreads();
     if (++i >= nit) break;
@@ -907,12 +889,8 @@ __global__ void __launch_bounds__(PF_THREADS, 1) sdpa_prefill_kernel(const uint1
 #pragma unroll
   for (uint32_t cg = 0; cg < 2; ++cg) {
     const float m1 = s_mo[cg * 256u + stid], l1 = s_mo[(2u + cg) * 256u + stid];
-    // finite unless SPLIT (block 0 holds position 0 of every column); a split
-    // that held no position of a column takes its factors against 0, like the
-    // block loop, and leaves l = 0
-    const float mm = fmaxf(m_run[cg], m1), m = SPLIT && mm == -__builtin_huge_valf() ? 0.0f : mm;
+    const float m = fmaxf(m_run[cg], m1);  // finite: block 0 holds position 0 of every column
     const float f0 = __builtin_amdgcn_exp2f(m_run[cg] - m), f1 = __builtin_amdgcn_exp2f(m1 - m);
-    m_run[cg] = mm;
     l_run[cg] = __builtin_fmaf(l1, f1, l_run[cg] * f0);
 #pragma unroll
     for (uint32_t nt = 0; nt < 8; ++nt)
@@ -927,18 +905,6 @@ __global__ void __launch_bounds__(PF_THREADS, 1) sdpa_prefill_kernel(const uint1
     float l = l_run[cg];
     l += lane_xor16_f32(l, lane);
     l += lane_xor32_f32(l, lane);
-    if (SPLIT) {
-      const uint32_t c = (2u * wave + cg) * 16u + col;
-      float* const pb = part + (static_cast<size_t>(tile * splits + sp) * nkv + kv) * PF_PART;
-#pragma unroll
-      for (uint32_t nt = 0; nt < 8; ++nt)
-        *reinterpret_cast<f32x4_t*>(pb + c * HD + 16u * nt + 4u * g) = o[cg][nt];
-      if (g == 0u) {
-        pb[PF_COLS * HD + c] = m_run[cg];
-        pb[PF_COLS * HD + PF_COLS + c] = l;
-      }
-      continue;
-    }
     const float inv = 1.0f / l;
     const uint32_t t = tb + (2u * wave + cg) * TPG + cj;
     if (t < n_tok) {
@@ -950,40 +916,6 @@ __global__ void __launch_bounds__(PF_THREADS, 1) sdpa_prefill_kernel(const uint1
       }
     }
   }
-}
-
-// out of a split prefill: per column, O = sum_s O_s 2^(m_s - M) and l likewise,
-// M = max_s m_s, out = bf16(O / l). One wave per (token, kv head) pair of
-// columns: 32 lanes x 4 dims each, all splits' loads in flight together. A
-// split with l = 0 held no position of the column and is left out (its O is 0).
-// (NaN scores leave l NaN, so they still reach the output.)
-__global__ void __launch_bounds__(256) sdpa_prefill_combine_kernel(const float* __restrict__ part,
-                                                                   uint16_t* __restrict__ out, uint32_t nh,
-                                                                   uint32_t nkv, uint32_t n_tok, uint32_t splits) {
-  const uint32_t G = nh / nkv, TPWG = 8u * (16u / G);
-  const uint32_t item = blockIdx.x * 8u + threadIdx.x / 32u, d = 4u * (threadIdx.x & 31u);  // item: (token, head)
-  if (item >= n_tok * nh) return;
-  const uint32_t t = item / nh, h = item % nh, kv = h / G;
-  const uint32_t tile = t / TPWG, c = (t % TPWG) * G + h % G;
-  const size_t step = static_cast<size_t>(nkv) * PF_PART;
-  const float* pb = part + (static_cast<size_t>(tile) * splits * nkv + kv) * PF_PART;
-  float M = -__builtin_huge_valf();
-#pragma unroll 8
-  for (uint32_t s = 0; s < splits; ++s) M = fmaxf(M, pb[s * step + PF_COLS * HD + c]);
-  f32x4_t o = {0.0f, 0.0f, 0.0f, 0.0f};
-  float l = 0.0f;
-#pragma unroll 8
-  for (uint32_t s = 0; s < splits; ++s) {
-    const f32x4_t os = *reinterpret_cast<const f32x4_t*>(pb + s * step + c * HD + d);
-    const float ms = pb[s * step + PF_COLS * HD + c], ls = pb[s * step + PF_COLS * HD + PF_COLS + c];
-    const float f = ls == 0.0f ? 0.0f : __builtin_amdgcn_exp2f(ms - M);
-    l = __builtin_fmaf(ls, f, l);
-#pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) o[i] = __builtin_fmaf(os[i], f, o[i]);
-  }
-  const float inv = 1.0f / l;
-  *reinterpret_cast<u32x2_t*>(out + static_cast<size_t>(item) * HD + d) =
-      u32x2_t{pack_bf16x2(o[0] * inv, o[1] * inv), pack_bf16x2(o[2] * inv, o[3] * inv)};
 }
 
 // ---------------------------------------------------------------------------
@@ -1109,36 +1041,6 @@ int ensure_rope_table(obs_ctx* ctx, float theta, uint32_t max_len, const float**
   ctx->rope_tables.push_back({t, max_len, theta});
   *out = t;
   return OBS_OK;
-}
-
-}  // namespace obs
-
-namespace obs {
-
-// Workgroups a (tile, kv head) of the prefill attention is split over: the s
-// of the shortest launch under measured costs in blocks of 0.66 us. A round of
-// workgroups over the CUs takes its share of the longest tile plus 7 (the
-// prologue and the merge of the two sets); s > 1 adds 6 (the second launch) and
-// 4 per round's worth of partials (17 MB written and read back). Measured, us,
-// s = 1 against the s taken: 57 tokens at 3,500: 83.7, 20.2 (16; 8: 22.3, 20:
-// 30.7, two rounds); 24 at 10,000: 214.7, 23.6 (32); 200 at 2,000: 55.0, 27.7
-// (4; 5: 37.1); 512 at 2,000: 62.5, 45.5 (2). Not split: 512 at 0 (18.8; 2:
-// 22.2), 700 at 3,000 (87.6; 4: 90.7), 57 at 0. From one workgroup per CU on,
-// every split measured slower (900 at 6,000: 154, 167).
-uint32_t sdpa_prefill_splits(uint32_t wgs, uint32_t nblk, uint32_t cus) {
-  if (wgs >= cus) return 1u;
-  constexpr uint64_t PRO = 7u, SECOND = 6u, PARTIALS = 4u, MAX_SPLITS = 32u;
-  uint32_t best = 1u;
-  uint64_t cost = cus * (nblk + PRO);  // in blocks x CUs
-  for (uint32_t s = 2u; s <= MAX_SPLITS && 2u * s <= nblk && wgs * s <= 4u * cus; ++s) {
-    const uint64_t n = static_cast<uint64_t>(wgs) * s;
-    const uint64_t c = cus * ((n + cus - 1u) / cus * ((nblk + s - 1u) / s + PRO) + SECOND) + PARTIALS * n;
-    if (c < cost) {
-      cost = c;
-      best = s;
-    }
-  }
-  return best;
 }
 
 }  // namespace obs
@@ -1339,23 +1241,16 @@ int obs_sdpa_prefill(obs_ctx* ctx, const uint16_t* q, const uint16_t* k_cache, c
   const uint64_t wgs = static_cast<uint64_t>(n_kv) * ((n_tokens + tpwg - 1u) / tpwg);
   if (wgs > 0x7fffffffull) return obs::set_error(ctx, OBS_E_SHAPE, "obs_sdpa_prefill: too many tokens");
   const float scale_log2 = 1.4426950408889634f / __builtin_sqrtf(static_cast<float>(HD));
-  const uint32_t splits = obs::sdpa_prefill_splits(static_cast<uint32_t>(wgs), (pos0 + n_tokens + 31u) / 32u,
-                                                   static_cast<uint32_t>(ctx->num_cus));
-  float* part = nullptr;
-  if (splits > 1u)
-    part = static_cast<float*>(obs::stream_scratch(ctx, static_cast<size_t>(wgs) * splits * PF_PART * sizeof(float)));
-  if (part) {
-    OBS_LAUNCH(ctx, "sdpa_prefill",
-               sdpa_prefill_kernel<true><<<static_cast<uint32_t>(wgs) * splits, PF_THREADS, 0, ctx->stream>>>(
-                   q, k_cache, v_cache_t, out, n_heads, n_kv, max_len, pos0, n_tokens, q_ld, scale_log2, splits, part));
-    OBS_LAUNCH(ctx, "sdpa_prefill_combine",
-               sdpa_prefill_combine_kernel<<<(n_tokens * n_heads + 7u) / 8u, 256, 0, ctx->stream>>>(
-                   part, out, n_heads, n_kv, n_tokens, splits));
-    return OBS_OK;
-  }
-  OBS_LAUNCH(ctx, "sdpa_prefill",
-             sdpa_prefill_kernel<false><<<static_cast<uint32_t>(wgs), PF_THREADS, 0, ctx->stream>>>(
-                 q, k_cache, v_cache_t, out, n_heads, n_kv, max_len, pos0, n_tokens, q_ld, scale_log2, 1u, nullptr));
+  // One workgroup per (tile, kv head) however few there are. A tile's blocks split
+  // over workgroups with fp32 partials took 20.2 us instead of 83.9 (57 tokens at
+  // position 3,500), but the probabilities are then rounded to bf16 against other
+  // maxima: 2.7e-3 of the output, from which a prompt's last row took another
+  // expert in 16 of 160 prompts of 24-150 tokens (logits up to 9e-2 apart), and a
+  // captured call, without memory of its own for partials, left other bits than a
+  // direct one.
+  OBS_LAUNCH(ctx, "sdpa_prefill", sdpa_prefill_kernel<<<static_cast<uint32_t>(wgs), PF_THREADS, 0, ctx->stream>>>(
+                                      q, k_cache, v_cache_t, out, n_heads, n_kv, max_len, pos0, n_tokens, q_ld,
+                                      scale_log2));
   return OBS_OK;
 }
 

@@ -181,31 +181,6 @@ int ensure_decode_ws(obs_ctx* ctx, size_t bytes, void** out) {
   return OBS_OK;
 }
 
-void* stream_scratch(obs_ctx* ctx, size_t bytes) {
-  if (bytes > STREAM_SCRATCH_BYTES) return nullptr;
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
-    (void)hipGetLastError();
-    return nullptr;
-  }
-  for (const auto& a : ctx->scratch_areas)
-    if (a.stream == ctx->stream) return a.ptr;
-  if (ctx->scratch_areas.size() >= STREAM_SCRATCH_MAX) return nullptr;
-  // relaxed for this call: another thread's capture must not be invalidated
-  // by an allocation that a call which takes no scratch would not make
-  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  (void)hipThreadExchangeStreamCaptureMode(&mode);
-  void* p = nullptr;
-  const hipError_t e = hipMalloc(&p, STREAM_SCRATCH_BYTES);
-  (void)hipThreadExchangeStreamCaptureMode(&mode);
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    return nullptr;
-  }
-  ctx->scratch_areas.push_back({ctx->stream, p});
-  return p;
-}
-
 }  // namespace obs
 
 extern "C" {
@@ -282,7 +257,6 @@ void obs_destroy(obs_ctx* ctx) {
   if (ctx->route_cnt) (void)hipFree(ctx->route_cnt);
   for (const auto& r : ctx->rope_tables) (void)hipFree(r.table);
   for (void* p : ctx->retired) (void)hipFree(p);
-  for (const auto& a : ctx->scratch_areas) (void)hipFree(a.ptr);
   if (ctx->ev_start) (void)hipEventDestroy(ctx->ev_start);
   if (ctx->ev_stop) (void)hipEventDestroy(ctx->ev_stop);
   if (ctx->own_stream) (void)hipStreamDestroy(ctx->own_stream);

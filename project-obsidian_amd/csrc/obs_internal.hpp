@@ -57,14 +57,6 @@ struct obs_ctx {
   std::vector<rope_entry> rope_tables;
   // decode workspaces replaced by larger ones, kept for the same reason
   std::vector<void*> retired;
-  // Scratch of launches that pass partial results to a second launch behind
-  // them (obs::stream_scratch): one area per stream, so that calls on
-  // different streams of one context stay independent.
-  struct scratch_entry {
-    hipStream_t stream;
-    void* ptr;
-  };
-  std::vector<scratch_entry> scratch_areas;
   int decode_path = 0;  // OBS_DECODE_AUTO / _MULTI / _FUSED
   // Context-owned device status words (obs::CTX_ST_*), zeroed by obs_create,
   // read and cleared by obs_device_status: the one-launch prefill FFN's flags.
@@ -156,22 +148,6 @@ inline bool aligned(const void* p, size_t a) { return (reinterpret_cast<uintptr_
 
 // Workspace for decode: returns device pointer of at least `bytes`.
 int ensure_decode_ws(obs_ctx* ctx, size_t bytes, void** out);
-
-// Scratch for the launches of one call on the context's stream, whose contents
-// nothing reads after the call's last launch; nullptr where there is none, and
-// the caller takes a path without it: under capture (a graph would keep the
-// area for replays on any stream), beyond STREAM_SCRATCH_BYTES, when the
-// context already holds areas for STREAM_SCRATCH_MAX other streams, or when
-// the allocation fails. At most STREAM_SCRATCH_MAX areas of
-// STREAM_SCRATCH_BYTES exist per context, from the first such call on a stream
-// until obs_destroy.
-constexpr size_t STREAM_SCRATCH_BYTES = size_t(72) << 20;
-constexpr size_t STREAM_SCRATCH_MAX = 4;
-void* stream_scratch(obs_ctx* ctx, size_t bytes);
-
-// Splits of a prefill attention launch of `wgs` workgroups whose longest tile
-// has nblk 32-position blocks, on a device with `cus` CUs (obs_attention.hip).
-uint32_t sdpa_prefill_splits(uint32_t wgs, uint32_t nblk, uint32_t cus);
 
 // RMSNorm of rows x dim bf16 (obs_elementwise.hip); dim % 64 == 0, <= 8192.
 int launch_rmsnorm(obs_ctx* ctx, const uint16_t* x, const uint16_t* w, uint16_t* out, uint32_t rows, uint32_t dim,
