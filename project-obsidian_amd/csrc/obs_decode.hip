@@ -43,8 +43,10 @@ __device__ __forceinline__ void load_words(const uint32_t* row, uint32_t lane, u
 
 // Sums of q_j * x_j over the 8 nibbles of w: even nibbles as the f16 subnormals
 // q * 2^-24, odd ones as q * 2^-20 (masked in place), each converted exactly
-// inside an fp32 fma. 13 instructions instead of dot8_q4's 19; the caller puts
-// the powers of two back (dot_mix_sum), which is exact.
+// inside an fp32 fma. 13 instructions instead of the 19 of a shift, mask and
+// conversion per nibble; the caller puts the powers of two back (dot_mix_sum).
+// Exact while q_j * x_j * 2^-24 is not below fp32's normal range: a chunk whose
+// values are all tiny is scaled first (mix_scale_up).
 struct DotMix {
   float a24, a20;
 };
@@ -60,9 +62,16 @@ __device__ __forceinline__ void dot8_q4_mix(uint32_t w, const float* x, DotMix& 
   d.a24 = fma_mix_f16<1>(p26, x[6], d.a24);
   d.a20 = fma_mix_f16<1>(p37, x[7], d.a20);
 }
-__device__ __forceinline__ float dot_mix_sum(const DotMix& d) {
-  return __builtin_fmaf(d.a20, 0x1p20f, d.a24 * 0x1p24f);
+__device__ __forceinline__ float dot_mix_sum(const DotMix& d, float unscale) {
+  return __builtin_fmaf(d.a20, 0x1p20f * unscale, d.a24 * (0x1p24f * unscale));
 }
+
+// The power of two that a lane's values of one chunk take before dot8_q4_mix,
+// from their largest magnitude: 2^90 where all of them are below 2^-98 (2^-24 of
+// that is 27 bits above fp32's smallest subnormal), else 1. Values that small
+// beside larger ones of the chunk lose nothing that its sum would keep.
+__device__ __forceinline__ float mix_scale_up(float largest) { return largest < 0x1p-98f ? 0x1p90f : 1.0f; }
+__device__ __forceinline__ float mix_scale_down(float largest) { return largest < 0x1p-98f ? 0x1p-90f : 1.0f; }
 
 constexpr uint32_t GU_WAVES = 4;
 constexpr uint32_t GU_WAVES_MAX = 2048;  // waves a gate/up launch aims at: 8 per CU
@@ -138,7 +147,7 @@ __global__ void __launch_bounds__(GU_WAVES * 64, 2) decode_gateup_kernel(
     }
     inv = 1.0f / __builtin_sqrtf(wave_sum_asc(ss) / static_cast<float>(H) + eps);
   }
-  float xf[CH * C], xs[CH];
+  float xf[CH * C], xs[CH], unscale[CH];
 #pragma unroll
   for (uint32_t j = 0; j < XQ; ++j) {
     const uint32_t d[4] = {xq[j].x, xq[j].y, xq[j].z, xq[j].w}, n[4] = {nq[j].x, nq[j].y, nq[j].z, nq[j].w};
@@ -154,6 +163,13 @@ __global__ void __launch_bounds__(GU_WAVES * 64, 2) decode_gateup_kernel(
     xs[c] = 0.0f;
 #pragma unroll
     for (uint32_t j = 0; j < C; ++j) xs[c] = xs[c] + xf[C * c + j];
+    float m = 0.0f;
+#pragma unroll
+    for (uint32_t j = 0; j < C; ++j) m = fmaxf(m, __builtin_fabsf(xf[C * c + j]));
+    const float up = mix_scale_up(m);
+    unscale[c] = mix_scale_down(m);
+#pragma unroll
+    for (uint32_t j = 0; j < C; ++j) xf[C * c + j] *= up;
   }
   float my_g = 0.0f, my_u = 0.0f;  // lane i < PR: the sums of row row0 + i
   bool mine = false;
@@ -168,8 +184,8 @@ __global__ void __launch_bounds__(GU_WAVES * 64, 2) decode_gateup_kernel(
         dot8_q4_mix(gq[i][W * c + j], xf + C * c + 8 * j, ag);
         dot8_q4_mix(uq[i][W * c + j], xf + C * c + 8 * j, au);
       }
-      pg = __builtin_fmaf(bf16_to_f32(sg[i][c]), dot_mix_sum(ag), __builtin_fmaf(bf16_to_f32(bg[i][c]), xs[c], pg));
-      pu = __builtin_fmaf(bf16_to_f32(su[i][c]), dot_mix_sum(au), __builtin_fmaf(bf16_to_f32(bu[i][c]), xs[c], pu));
+      pg = __builtin_fmaf(bf16_to_f32(sg[i][c]), dot_mix_sum(ag, unscale[c]), __builtin_fmaf(bf16_to_f32(bg[i][c]), xs[c], pg));
+      pu = __builtin_fmaf(bf16_to_f32(su[i][c]), dot_mix_sum(au, unscale[c]), __builtin_fmaf(bf16_to_f32(bu[i][c]), xs[c], pu));
     }
     pg = wave_sum_asc(pg);
     pu = wave_sum_asc(pu);
@@ -201,6 +217,7 @@ __global__ void __launch_bounds__(DN_WAVES * 64, 2) decode_down_kernel(
     const uint16_t* __restrict__ residual, uint16_t* __restrict__ y, uint32_t n_exp, uint32_t k,
     uint32_t H, uint32_t I, uint32_t group) {
   __shared__ float4 s_h[NC * 8 * 64];
+  __shared__ float s_un[NC * 64];  // per chunk: what undoes its scaling (mix_scale_up)
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t o = __builtin_amdgcn_readfirstlane(blockIdx.x * DN_WAVES + tid / 64u);  // < H (H % 8 == 0)
   const uint32_t cpr = I / 32u, nch = k * cpr;  // chunks of an expert's row, of an output row
@@ -234,12 +251,21 @@ __global__ void __launch_bounds__(DN_WAVES * 64, 2) decode_down_kernel(
 #pragma unroll
   for (int i = 0; i < NC; ++i) {
     const uint32_t f = tid + 512u * i, c = f / 8u, j = f % 8u;  // float4 j of chunk c
-    s_h[(c / 64u * 8u + j) * 64u + ((c % 64u) ^ j)] = hv[i];    // (past nch: a copy of the last, never used)
+    float m = fmaxf(fmaxf(__builtin_fabsf(hv[i].x), __builtin_fabsf(hv[i].y)),
+                    fmaxf(__builtin_fabsf(hv[i].z), __builtin_fabsf(hv[i].w)));
+    m = fmaxf(m, dpp_f32<DPP_XOR1>(m));  // over the chunk's 8 lanes
+    m = fmaxf(m, dpp_f32<DPP_XOR2>(m));
+    m = fmaxf(m, dpp_f32<DPP_HALF_MIRROR>(m));
+    const float up = mix_scale_up(m);
+    const float4 v = make_float4(hv[i].x * up, hv[i].y * up, hv[i].z * up, hv[i].w * up);
+    s_h[(c / 64u * 8u + j) * 64u + ((c % 64u) ^ j)] = v;  // (past nch: a copy of the last, never used)
+    if (j == 0u) s_un[c] = mix_scale_down(m);
   }
   __syncthreads();
   float acc = 0.0f;
 #pragma unroll
   for (int i = 0; i < NC; ++i) {
+    const float unscale = s_un[64 * i + lane];
     float hf[32], hs = 0.0f;
 #pragma unroll
     for (uint32_t j = 0; j < 8; ++j) {
@@ -252,7 +278,7 @@ __global__ void __launch_bounds__(DN_WAVES * 64, 2) decode_down_kernel(
     dot8_q4_mix(q[i].y, hf + 8, a);
     dot8_q4_mix(q[i].z, hf + 16, a);
     dot8_q4_mix(q[i].w, hf + 24, a);
-    const float part = __builtin_fmaf(bf16_to_f32(sc[i]), dot_mix_sum(a), bf16_to_f32(bi[i]) * hs);
+    const float part = __builtin_fmaf(bf16_to_f32(sc[i]), dot_mix_sum(a, unscale), bf16_to_f32(bi[i]) * (hs * unscale));
     acc = ok[i] ? __builtin_fmaf(wr[i], part, acc) : acc;
   }
   acc = wave_sum_asc(acc);

@@ -126,6 +126,43 @@ def test_decode_multi_row_splits(exe, E, H, I, K, norm):
     assert np.all(np.abs(got - ref) <= 2.0 ** -8 * np.abs(ref) + 1e-5 * np.sqrt(np.mean(ref ** 2)))
 
 
+@pytest.mark.parametrize("where", ["x", "h"])
+@pytest.mark.parametrize("E,H,I,K", [(8, 1024, 512, 4), (8, 2048, 768, 7), (8, 4096, 2048, 6)])
+def test_decode_multi_tiny_values(exe, E, H, I, K, where):
+    """Activations (or h) near the bottom of fp32's range, with scales that bring
+    the outputs back to order one: the sums keep fp32's relative precision. In
+    the second half of the columns they are of the usual size, and of no weight
+    (scales of 2^-126), so one wave meets both."""
+    t = synth.moe_layer(90 + H, E, H, I, 64)
+
+    def mul(key, e):
+        v = synth.bf16_bits_to_f32(t[key]).astype(np.float64) * np.exp2(e)
+        t[key] = synth.f32_to_bf16_bits(v.astype(np.float32))
+    x = synth.bf16_normal(np.random.default_rng(H + I), H)
+    if where == "x":
+        e = np.where(np.arange(H // 64) < H // 128, 124.0, -126.0)
+        for key in ("gate_s", "gate_b", "up_s", "up_b"):
+            mul(key, e)
+        x = synth.f32_to_bf16_bits(synth.bf16_bits_to_f32(x) * np.float32(2.0 ** -126) *
+                                   np.where(np.arange(H) < H // 2, 1.0, 2.0 ** 126).astype(np.float32))
+    else:
+        rows = np.where(np.arange(I) < I // 2, -64.0, 0.0)[:, None]
+        for key in ("gate_s", "gate_b", "up_s", "up_b"):
+            mul(key, rows)
+        e = np.where(np.arange(I // 64) < I // 128, 120.0, -126.0)
+        for key in ("down_s", "down_b"):
+            mul(key, e)
+    layer, L = oh.MoeLayer.upload(exe, t), O.Layer(t, E, H, I, 64)
+    cfg = oh.MoeConfig(E, K, H, I, 64, True)
+    got, gi, gw = _decode(exe, cfg, layer, x, oh.OBS_DECODE_MULTI)
+    _, ri, rw = O.router(L, x, K, True)
+    assert np.array_equal(gi, ri[0])
+    want = O.moe_decode(L, x, K, True, ids=ri, w=rw)[0][0]
+    assert 1e-6 < np.sqrt(np.mean(want ** 2)) < 1e9
+    # half a unit of 8 bits; h in fp32 subnormals of 2^-149 has 17 bits or more of its largest value
+    assert np.all(np.abs(_f32(got) - want) <= 2.0 ** -8 * np.abs(want) + 1e-4 * np.sqrt(np.mean(want ** 2)))
+
+
 @pytest.mark.parametrize("E,H,I,K,T", [(256, 2048, 768, 8, 96), (64, 2048, 768, 8, 130), (32, 1024, 512, 4, 77)])
 def test_prefill_shapes(exe, E, H, I, K, T):
     t = synth.moe_layer(40 + E + H, E, H, I, 64)
