@@ -235,6 +235,7 @@ int obs_create(int device, obs_ctx** out) {
   }
   if (rc == OBS_OK) rc = obs::probe_dispatch(ctx);
   if (rc == OBS_OK) rc = obs::prefill_init(ctx);
+  if (rc == OBS_OK) rc = obs::router_init(ctx);
   if (rc != OBS_OK) {
     g_create_error = serr.empty() ? ctx->err : serr;
     obs_destroy(ctx);

@@ -156,6 +156,7 @@ int launch_rmsnorm(obs_ctx* ctx, const uint16_t* x, const uint16_t* w, uint16_t*
 // The router step (obs_router.hip): logits, then routing. norm_w (with eps):
 // the rows are normalised first, as launch_rmsnorm does; only where
 // route_one_launch() says that the step is one launch (nullptr elsewhere).
+int router_init(obs_ctx* ctx);  // at obs_create
 bool route_one_launch(const obs_ctx* ctx, uint32_t T);
 int launch_route(obs_ctx* ctx, const uint32_t* w8, const uint16_t* s, const uint16_t* b, const uint16_t* x,
                  float* logits, int32_t* ids, float* w, uint32_t T, uint32_t in, uint32_t n_exp, uint32_t group,

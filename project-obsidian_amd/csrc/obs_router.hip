@@ -30,7 +30,7 @@ using namespace obsd;
 
 constexpr uint32_t ROUTE_FUSED_TOKENS = 8;
 
-// ---- logits of more than 64 tokens, on the matrix cores ----------------------
+// ---- logits of many tokens, on the matrix cores (logits_by_rows: the line) ----
 // A lane's partial of the reduction order above is a chain of in/64 fp32 fmas over
 // consecutive columns. v_mfma_f32_16x16x1_4b_f32 is one such fma (correctly
 // rounded, subnormals kept: checked bit for bit) for each (token, expert) of four
@@ -119,7 +119,9 @@ __global__ void __launch_bounds__(64 * LG_WAVES, C <= 32u ? 4 : 2)
   // a tile's logits from the waves' partials
   auto finish = [&](uint32_t tl) __attribute__((always_inline)) {
     if (tid < LG_TILE * LG_TILE) {
-      const uint32_t t = tl * LG_TILE + tid / LG_TILE, e = e0 + tid % LG_TILE;
+      const uint32_t t = tl * LG_TILE + tid / LG_TILE;
+      uint32_t e = e0 + tid % LG_TILE;
+      asm("" : "+v"(e));  // the address is formed here: kept over the tiles it went to scratch
       const float v = ((s_part[0][tid] + s_part[1][tid]) + (s_part[2][tid] + s_part[3][tid])) +
                       ((s_part[4][tid] + s_part[5][tid]) + (s_part[6][tid] + s_part[7][tid]));
       if (t < T && e < n_exp) logits[static_cast<uint64_t>(t) * n_exp + e] = v;
@@ -164,7 +166,7 @@ __global__ void __launch_bounds__(64 * LG_WAVES, C <= 32u ? 4 : 2)
   finish(tile - 8u * slots);
 }
 
-// ---- up to 64 tokens, and the one-launch router of up to 8 --------------------
+// ---- few tokens, and the one-launch router of up to 8 -------------------------
 // The routing step of the one-launch router (obs_route): where the range's
 // ids and weights go, and the per-range counters that elect the workgroup
 // that routes (context memory, zero between launches); with NORM the RMSNorm
@@ -194,11 +196,8 @@ struct RouteTail {
 // per-token wave). NQ: logit slots per lane when routing.
 // NORM: each workgroup normalises the rows as it stages them, in obs_rmsnorm's
 // sequence, so a decode layer needs no launch for the norm.
-// FUSED off: the logits of 9 to 64 tokens alone, workgroup (x, y) the rows 4x.. and
-// the tokens 8y.. (the matrix kernel above has a tile's 2.1 us of instructions in
-// one workgroup whatever the number of tokens: with the top-k launch 37 tokens 11.5
-// us, this one 9.8; 64: 11.6 and 10.0; from 65 on the matrix kernel, 128: 11.6 and
-// 12.5).
+// FUSED off: the logits of few tokens alone, workgroup (x, y) the rows 4x.. and
+// the tokens 8y..
 template <int WPL, int NQ, bool NORM, bool FUSED>
 __global__ void __launch_bounds__(256) route_rows_kernel(const uint32_t* __restrict__ w8,
                                                          const uint16_t* __restrict__ s,
@@ -394,12 +393,40 @@ int check_router_shape(obs_ctx* ctx, const char* who, uint32_t in, uint32_t n_ex
   return OBS_OK;
 }
 
+// Whether T tokens' logits take the kernel of few tokens: while its workgroups (4
+// experts x 8 tokens each) fit the GPU at once, two to a CU up to in = 2048 and one
+// at 4096. The matrix kernel has a tile's instructions in one workgroup whatever the
+// number of tokens. Measured, us, matrix kernel | this one, 128 experts: in = 2048
+// 64 tokens 6.5 | 5.0, 128 (512 workgroups) 6.5 | 5.7, 160 6.6 | 6.8; in = 4096 64
+// tokens (256 workgroups) 10.3 | 8.6, 72 10.3 | 12.0; 256 experts: in = 2048 64
+// tokens 6.5 | 5.7, 72 6.5 | 6.8; in = 4096 32 tokens 10.3 | 8.5, 48 10.3 | 12.1.
+// (At 512 and 1,024 columns it stays ahead to twice as many.)
+bool logits_by_rows(const obs_ctx* ctx, uint32_t T, uint32_t in, uint32_t n_exp) {
+  const uint64_t wgs = ((n_exp + 3u) / 4u) * ((static_cast<uint64_t>(T) + ROUTE_FUSED_TOKENS - 1u) / ROUTE_FUSED_TOKENS);
+  return wgs <= static_cast<uint64_t>(ctx->num_cus) * (in <= 2048u ? 2u : 1u);
+}
+
+// The matrix kernel's staged tiles are more than 64 KB from in = 2048 on: its
+// limit is raised once per context, at creation.
+int router_init(obs_ctx* ctx) {
+  const struct {
+    const void* fn;
+    size_t lds;
+  } ks[] = {{reinterpret_cast<const void*>(&gate_logits_mfma_kernel<32u, true>), lg_lds_bytes<32u>()},
+            {reinterpret_cast<const void*>(&gate_logits_mfma_kernel<32u, false>), lg_lds_bytes<32u>()},
+            {reinterpret_cast<const void*>(&gate_logits_mfma_kernel<64u, true>), lg_lds_bytes<64u>()},
+            {reinterpret_cast<const void*>(&gate_logits_mfma_kernel<64u, false>), lg_lds_bytes<64u>()}};
+  for (const auto& k : ks)
+    OBS_HIP_TRY(ctx, hipFuncSetAttribute(k.fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(k.lds)));
+  return OBS_OK;
+}
+
 // One workgroup per CU (two up to in = 2048, by LDS and registers), each running
 // its share of the token tiles.
 int launch_gate_logits(obs_ctx* ctx, const uint32_t* w8, const uint16_t* s, const uint16_t* b,
                        const uint16_t* x, float* logits, uint32_t T, uint32_t in, uint32_t n_exp,
                        uint32_t group) {
-  if (T <= 8u * ROUTE_FUSED_TOKENS) {
+  if (logits_by_rows(ctx, T, in, n_exp)) {
     const dim3 grid((n_exp + 3) / 4, (T + ROUTE_FUSED_TOKENS - 1u) / ROUTE_FUSED_TOKENS);
     const size_t lds = sizeof(uint16_t) * ROUTE_FUSED_TOKENS * in;
     const RouteTail none{};

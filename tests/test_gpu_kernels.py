@@ -110,11 +110,16 @@ def test_q8_gate_logits_other_widths_bit_exact(exe, H, E, T):
         assert np.array_equal(got[t].view(np.uint32), ref.view(np.uint32)), f"token {t}"
 
 
-# The matrix-core logits (from 65 tokens): each width, the last tile of tokens and of
-# experts partly filled, groups shorter than a lane's columns, several tiles per
-# workgroup (over 1,024 tokens at 128 experts, 512 at 256).
+# Both logits kernels: the one of few tokens up to the last size it takes (512
+# workgroups of 4 experts x 8 tokens, 256 at width 4,096), the matrix-core one from
+# the next and well past it. Each width, the last tile of tokens and of experts
+# partly filled, groups shorter than a lane's columns, several tiles per workgroup
+# (over 1,024 tokens at 128 experts, 512 at 256).
 @pytest.mark.parametrize("H,E,T,group", [(512, 60, 65, 64), (512, 16, 129, 4), (1024, 128, 80, 8), (2048, 17, 97, 16),
-                                         (2048, 256, 700, 64), (4096, 33, 130, 32), (4096, 128, 600, 64)])
+                                         (2048, 256, 700, 64), (4096, 33, 130, 32), (4096, 128, 600, 64),
+                                         (2048, 128, 128, 64), (2048, 128, 129, 64), (4096, 128, 64, 64),
+                                         (4096, 128, 65, 64), (512, 60, 700, 4), (512, 256, 601, 64),
+                                         (1024, 128, 401, 8), (2048, 17, 1700, 16), (4096, 33, 497, 32)])
 def test_q8_gate_logits_tiles_bit_exact(exe, H, E, T, group):
     """Bit for bit the reduction order, also where sums go through subnormals."""
     rng = np.random.default_rng(320 + H + E + T)
