@@ -28,7 +28,10 @@ from typing import Dict, Optional, Tuple
 
 PKG = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
-# kernel -> (pattern of its rocprofv3 name, the sources it is compiled from)
+_PREFILL = ("csrc/obs_prefill.hip", "csrc/obs_q4_dequant.hpp", "csrc/obs_internal.hpp")
+
+# kernel -> (pattern of its rocprofv3 name, the sources it is compiled from: its
+# file and the headers that file includes)
 KERNELS = {
     "decode_fused": (r"decode_fused_kernel<2, false>",
                      ("csrc/obs_decode_fused.hip", "csrc/obs_moe_half.hpp", "csrc/obs_internal.hpp")),
@@ -37,11 +40,11 @@ KERNELS = {
     "layer_fused": (r"layer_fused_kernel<2>",
                     ("csrc/obs_layer_fused.hip", "csrc/obs_attn_half.hpp", "csrc/obs_moe_half.hpp",
                      "csrc/obs_internal.hpp")),
-    "grouped_gemm_gateup": (r"grouped_gemm_kernel<1u, 3u>", ("csrc/obs_prefill.hip", "csrc/obs_internal.hpp")),
-    "grouped_gemm_down": (r"grouped_gemm_kernel<2u, 5u>", ("csrc/obs_prefill.hip", "csrc/obs_internal.hpp")),
-    "moe_ffn": (r"moe_ffn_kernel<2u>", ("csrc/obs_prefill.hip", "csrc/obs_internal.hpp")),
-    "moe_group": (r"group_kernel<", ("csrc/obs_prefill.hip",)),
-    "moe_combine": (r"combine_kernel", ("csrc/obs_prefill.hip",)),
+    "grouped_gemm_gateup": (r"grouped_gemm_kernel<1u, 3u>", _PREFILL),
+    "grouped_gemm_down": (r"grouped_gemm_kernel<2u, 5u>", _PREFILL),
+    "moe_ffn": (r"moe_ffn_kernel<2u>", _PREFILL),
+    "moe_group": (r"group_kernel<", _PREFILL),
+    "moe_combine": (r"(?<!\w)combine_kernel", _PREFILL),
 }
 COPY = r"copyBuffer"
 
@@ -73,7 +76,7 @@ def _short(name: str) -> Optional[str]:
     if re.search(COPY, name):
         return "__copy"
     for k, (pat, _) in KERNELS.items():
-        if re.search(re.escape(pat) if "<" in pat else pat, name):
+        if re.search(pat if pat.startswith("(?") else re.escape(pat), name):
             return k
     return None
 

@@ -4,6 +4,9 @@ digest of each kernel's sources, which bench.py compares before it reports a
 traffic figure."""
 import csv
 import os
+import re
+
+import pytest
 
 import obsidian_hip.profiles as P
 
@@ -37,6 +40,30 @@ def test_digest_follows_the_sources():
     assert a == P.source_digest("grouped_gemm_down")  # one source file holds both
     assert a != P.source_digest("decode_fused") and P.source_digest("nope") is None
     assert all(os.path.exists(os.path.join(P.PKG, f)) for _, fs in P.KERNELS.values() for f in fs)
+
+
+@pytest.mark.parametrize("kernel", P.KERNELS)
+def test_digest_covers_the_included_headers(kernel):
+    """A kernel's sources are its file and every header of csrc/ that it includes, directly or not."""
+    todo, seen = [P.KERNELS[kernel][1][0]], set()
+    while todo:
+        f = todo.pop()
+        seen.add(f)
+        with open(os.path.join(P.PKG, f)) as src:
+            inc = ["csrc/" + n for n in re.findall(r'^#include "(\w+\.hpp)"', src.read(), re.M)]
+        todo += [n for n in inc if n not in seen]
+    assert set(P.KERNELS[kernel][1]) == seen
+
+
+@pytest.mark.parametrize("name,kernel", [
+    ("void (anonymous namespace)::combine_kernel(unsigned short const*, int const*)", "moe_combine"),
+    ("(anonymous namespace)::combine_kernel(unsigned short const*)", "moe_combine"),
+    ("void (anonymous namespace)::sdpa_combine_kernel(float const*)", None),
+    ("void (anonymous namespace)::sdpa_prefill_combine_kernel(float const*)", None),
+    ("void (anonymous namespace)::group_kernel<true>(int const*)", "moe_group"),
+    ("void (anonymous namespace)::moe_ffn_kernel<2u>(GemmArgs, GemmArgs, FfnSync)", "moe_ffn")])
+def test_kernel_names(name, kernel):
+    assert P._short(name) == kernel
 
 
 def test_mfma_util_fractions(tmp_path):
