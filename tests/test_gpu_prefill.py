@@ -157,8 +157,9 @@ def test_q4_matmul_few_rows(exe, T, in_f, out_f):
                                                (1889, 2048, 5120, True)])
 def test_q4_matmul_few_rows_operand_bit_exact(exe, T, in_f, out_f, huge):
     """As test_q4_matmul_weight_operand_bit_exact, at a projection's width and from
-    half a tile to 15: row t is one-hot at column (37 t) % in_f, so Y[t] is that
-    column of the bf16 weight operand."""
+    half a tile to 15 (the 256-column form from 13 tiles on, 128 columns before):
+    row t is one-hot at column (37 t) % in_f, so Y[t] is that column of the bf16
+    weight operand."""
     rng = np.random.default_rng(4300 + T + huge)
     w = rng.integers(0, 2**32, size=(out_f, in_f // 8), dtype=np.uint64).astype(np.uint32)
     s, b = _extreme_scales(rng, out_f, in_f // 64, huge)
@@ -218,6 +219,32 @@ def test_moe_prefill_zipf_vs_oracle(exe, qwen, T, seed):
     rel_bf = _close(y, ref_bf, BF_NORM, BF_ELEM)
     rel64 = _close(y, ref64, 1e-2)
     print(f"T={T}: rel vs bf16-operand oracle {rel_bf:.2e}, vs fp64 oracle {rel64:.2e}")
+
+
+@pytest.mark.parametrize("inorder", [True, False])  # the expert FFN in one launch, in two
+@pytest.mark.parametrize("proj", ["gate", "up", "down"])
+def test_moe_prefill_scale_beyond_fast_dequant(exe, proj, inorder):
+    """One scale of 2^110 (the in-place nibble dequantization ends at 2^100) in
+    one row of one expert: its tile takes the reference form, in each GEMM."""
+    e, k, h, i, T = 8, 2, 1024, 256, 150
+    t = synth.moe_layer(37, e, h, i, 64)
+    t[proj + "_s"][3, 130, -1] = 0x7680  # 2^110
+    layer, L = oh.MoeLayer.upload(exe, t), O.Layer(t, e, h, i, 64)
+    X = synth.bf16_normal(np.random.default_rng(38), (T, h))
+    ids, w = synth.zipf_routing(T, e, k, 0.5, seed=39)
+    assert np.any(ids == 3) and np.any(np.all(ids != 3, axis=1))
+    _, xcd_map, inorder_ok = exe.dispatch_info()
+    kernels = {}
+    try:
+        exe.set_dispatch_facts(xcd_map, inorder_ok and inorder)
+        got = _f32(_prefill(exe, oh.MoeConfig(e, k, h, i, 64, True), layer, X, ids, w, kernels=kernels))
+    finally:
+        exe.set_dispatch_facts(xcd_map, inorder_ok)
+    assert ("moe_ffn" in kernels) == (inorder and inorder_ok)
+    ref = O.moe_prefill(L, X, ids, w, O.MODE_MFMA_BF16)
+    assert np.max(np.abs(ref)) > 2.0 ** 90 and np.all(np.isfinite(got))
+    floor = 1e-2 * np.median(np.abs(ref), axis=1, keepdims=True)  # of the token's outputs, not of the huge one
+    assert np.all(np.abs(got - ref) <= 1e-2 * np.abs(ref) + floor)
 
 
 def test_moe_prefill_many_tiles_even_split(exe):
