@@ -123,7 +123,7 @@ def bench_decode(torch, oh, exe, args):
     # is the timed region (HIP events on the context's stream around the graph
     # replays) divided by the launches in it; the per-launch event pairs above
     # add the event records' own overhead and are reported beside it. The
-    # 4-launch path's largest kernel is gate/up, timed by its event pairs.
+    # several-launch path's largest kernel is gate/up, timed by its event pairs.
     roof = None
     if "decode_fused" in kernels:
         name, nbytes, us = "decode_fused", LAYER_BYTES, us_layer

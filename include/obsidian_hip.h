@@ -264,14 +264,15 @@ typedef struct obs_moe_layer {
  * free for that launch (no other kernel holding them). A wait that times out
  * is reported by obs_device_status(): call it after a sequence of calls (or a
  * graph replay) before using their outputs. Other shapes, and devices with
- * fewer CUs, run as 4 launches. */
+ * fewer CUs, run as 3 launches (router with the norm, gate/up, down; up to 5
+ * where the router is not one launch). */
 int obs_moe_decode(obs_ctx* ctx, const obs_moe_config* cfg, const obs_moe_layer* layer,
                    const uint16_t* x, const uint16_t* residual, uint16_t* y,
                    int32_t* ids_out, float* w_out);
 
 /* obs_moe_decode without any allocation: the same kernels, results and path
  * choice, with every intermediate (the fused path's exchange area, the
- * 4-launch path's logits, routing, h and normalised x) in a file-scope device
+ * several-launch path's logits, routing, h and normalised x) in a file-scope device
  * array of 272,896 bytes that each GPU holds for the life of the process
  * (looked up per device by obs_create). It calls no hipMalloc, hipFree or
  * allocating routine, so it may run under HIP graph capture without a warm-up

@@ -11,7 +11,7 @@ namespace {
 thread_local std::string g_create_error;
 
 // The scratch of obs_moe_decode_static (the fused decode's exchange area and
-// the 4-launch path's intermediates), a file-scope device array: every GPU the
+// the several-launch path's intermediates), a file-scope device array: every GPU the
 // library runs on holds its own copy until the process ends. Host code never
 // passes `scratch` itself to a kernel (on the host it is only a stand-in for
 // the symbol): obs_create looks up each device's address once, with that

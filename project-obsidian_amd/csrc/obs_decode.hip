@@ -6,8 +6,8 @@
 // (disk_io.rs:79-102, forward.rs:431-435) and issues 5 dispatches per expert;
 // here the whole expert table is resident in HBM (stacked [E, ...] tensors)
 // and the layer runs as 3 launches: router (with the post-attention norm),
-// gate/up+SwiGLU, down+combine (two or three more where the router is not one
-// launch). Weights are read exactly once with 16-byte coalesced loads.
+// gate/up+SwiGLU, down+combine (one or two more where the router is not one
+// launch: its top-k and the norm). Weights are read exactly once with 16-byte coalesced loads.
 //
 // Numerics: dots accumulate in fp32 using the per-group factored form
 //   sum_c (q_c*s + b) * x_c = s * sum_c q_c*x_c + b * sum_c x_c
@@ -82,11 +82,12 @@ constexpr uint32_t GU_WAVES_MAX = 2048;  // waves a gate/up launch aims at: 8 pe
 //
 // Bound by HBM: k * I * H weights of both matrices at 4.5 bits. Every wave
 // requests all of its rows at once (6 row pairs of H = 4096 are 24 KB a wave, 196
-// KB in flight per CU) and there is no second round of waves, so the first rows'
-// dots run while the last are on their way; twice the waves of 3 rows measured
-// 20.1 us against 18.3. E 16, H 4096, I 2048, k 6 (57 MB): 20.3 us with 2 rows a
-// wave, 22.2 with 6 and dot8_q4 over 64 contiguous columns a lane, 18.3 us (3.1
-// TB/s) as it is.
+// KB in flight per CU), so the first rows' dots run while the last are on their
+// way. Up to 12,288 row pairs (k 6, I 2048) all waves of an H = 4096 launch are
+// resident at once, with 8 to a CU; at k 8, I 2048 a third of them run in a second
+// round. E 16, H 4096, I 2048, k 6 (57 MB): 20.3 us with 2 rows a wave, 20.1 with 3,
+// 22.2 with 6 and a shift-and-convert dot product over 64 contiguous columns a
+// lane, 18.8 with the one below, 19.2 (3.0 TB/s) with its scaling of tiny chunks.
 // NORM: x is normalised first, in obs_rmsnorm's sequence (its sum of squares over
 // the columns a lane owns there), so no launch of its own is needed (4.6 us).
 template <int W, int CH, int PR, bool NORM>
@@ -204,10 +205,11 @@ __global__ void __launch_bounds__(GU_WAVES * 64, 2) decode_gateup_kernel(
 // Bound by HBM (k * I * H weights): a wave requests all of its weights before it
 // uses the first. h is staged in LDS in the order the lanes read it
 // ([chunk / 64][float4][lane], the lane xor-ed with the float4's index so that the
-// stores of one chunk's 8 float4 spread over the banks). E 16, H 4096, I 2048, k 6
-// (28 MB): 10.1 us (11.1 with two output rows per wave, which reads h half as
-// often). A lane that kept the I / 8 values of its part of a rank's h in registers
-// spilled them from I = 1,024 on: 72.5 us.
+// stores of one chunk's 8 float4 spread over the banks), where the chunk's scaling
+// of tiny values is also done once for the 8 waves. E 16, H 4096, I 2048, k 6 (28
+// MB): 10.4 us (10.1 without that scaling; 11.1 with two output rows per wave, which
+// reads h half as often). A lane that kept the I / 8 values of its part of a rank's
+// h in registers spilled them from I = 1,024 on: 72.5 us.
 constexpr uint32_t DN_WAVES = 8;
 
 template <int NC>
@@ -372,7 +374,7 @@ int launch_decode_experts(obs_ctx* ctx, const obs_moe_config* cfg, const obs_moe
 }
 
 // Validates a decode call and picks its path (the one-launch fused kernel, or
-// the 4 launches).
+// the several launches).
 int decode_plan(obs_ctx* ctx, const char* who, const obs_moe_config* cfg, const obs_moe_layer* layer,
                 const uint16_t* x, const uint16_t* y, bool* fused) {
   int rc = check_moe_config(ctx, who, cfg);
@@ -397,14 +399,14 @@ int decode_plan(obs_ctx* ctx, const char* who, const obs_moe_config* cfg, const 
   return OBS_OK;
 }
 
-// Workspace of the 4-launch path: logits [E] | ids [k] | w [k] | h [k, I] | normed x [H].
+// Workspace of the several-launch path: logits [E] | ids [k] | w [k] | h [k, I] | normed x [H].
 size_t multi_ws_bytes(const obs_moe_config* cfg) {
   return align256(sizeof(float) * cfg->n_exp) + align256(sizeof(int32_t) * cfg->top_k) +
          align256(sizeof(float) * cfg->top_k) + align256(sizeof(float) * cfg->top_k * cfg->inter) +
          align256(sizeof(uint16_t) * cfg->hidden);
 }
 
-// The 4-launch path over a workspace of multi_ws_bytes(cfg) at `base`.
+// The several-launch path over a workspace of multi_ws_bytes(cfg) at `base`.
 int decode_multi(obs_ctx* ctx, const obs_moe_config* cfg, const obs_moe_layer* layer, const uint16_t* x,
                  const uint16_t* residual, uint16_t* y, int32_t* ids_out, float* w_out, char* base) {
   const uint32_t E = cfg->n_exp, k = cfg->top_k, H = cfg->hidden, I = cfg->inter;

@@ -89,7 +89,7 @@ namespace obs {
 
 // The scratch of obs_moe_decode_static: one file-scope device array per GPU
 // (obs_context.hip), the fused decode's exchange area followed by the
-// 4-launch path's logits / ids / weights / h / normalised x at the largest
+// several-launch path's logits / ids / weights / h / normalised x at the largest
 // shape obs_moe_decode accepts (E 256, top_k 8, inter 2048, hidden 4096).
 constexpr size_t STATIC_FUSED_BYTES = 197632;
 constexpr size_t STATIC_MULTI_BYTES = 1024 + 256 + 256 + 8 * 2048 * 4 + 4096 * 2;
@@ -283,23 +283,6 @@ __device__ __forceinline__ float silu_mul(float g, float u) { return (g / (1.0f 
 __device__ __forceinline__ float silu_mul_fast(float g, float u) {
   const float e = __builtin_amdgcn_exp2f(-g * 1.44269504088896341f);
   return (g * __builtin_amdgcn_rcpf(1.0f + e)) * u;
-}
-
-// Sum over the 8 nibbles of `w` of q_j * x[j] (nibble j = (w >> 4j) & 15),
-// fp32 fma chain in nibble order. The nibbles are split into the bytes of two
-// words so each converts with one byte-to-float instruction.
-__device__ __forceinline__ float dot8_q4(uint32_t w, const float* x, float acc) {
-  const uint32_t lo = w & 0x0f0f0f0fu;         // nibbles 0,2,4,6 in bytes 0..3
-  const uint32_t hi = (w >> 4) & 0x0f0f0f0fu;  // nibbles 1,3,5,7
-  acc = __builtin_fmaf(static_cast<float>(lo & 0xffu), x[0], acc);
-  acc = __builtin_fmaf(static_cast<float>(hi & 0xffu), x[1], acc);
-  acc = __builtin_fmaf(static_cast<float>((lo >> 8) & 0xffu), x[2], acc);
-  acc = __builtin_fmaf(static_cast<float>((hi >> 8) & 0xffu), x[3], acc);
-  acc = __builtin_fmaf(static_cast<float>((lo >> 16) & 0xffu), x[4], acc);
-  acc = __builtin_fmaf(static_cast<float>((hi >> 16) & 0xffu), x[5], acc);
-  acc = __builtin_fmaf(static_cast<float>(lo >> 24), x[6], acc);
-  acc = __builtin_fmaf(static_cast<float>(hi >> 24), x[7], acc);
-  return acc;
 }
 
 // ---- DPP cross-lane primitives (gfx9 DPP controls) -------------------------

@@ -86,7 +86,7 @@ int obs_layer_decode(obs_ctx* ctx, const obs_attn_layer* attn, const obs_moe_con
                           "%s: needs hidden 2048, inter 768, top_k 8, group 64, n_exp <= 256 and a post-attention "
                           "norm weight", who);
   if (ctx->decode_path == OBS_DECODE_MULTI)
-    return obs::set_error(ctx, OBS_E_UNSUPPORTED, "%s: the context is set to the 4-launch decode path", who);
+    return obs::set_error(ctx, OBS_E_UNSUPPORTED, "%s: the context is set to the several-launch decode path", who);
   if (!(obs::dispatch_gate(ctx->num_cus, ctx->xcd_map_ok, ctx->inorder_ok) & OBS_PATH_FUSED_DECODE))
     return obs::set_error(ctx, OBS_E_UNSUPPORTED, "%s: the device's dispatch does not allow the one-launch MoE half",
                           who);

@@ -108,7 +108,7 @@ class Model:
         """Whether the MoE half can share the attention half's launch
         (obs_layer_decode): the one-launch MoE shape (hidden 2048, inter 768,
         top-8, group 64, at most 256 experts) on a device whose dispatch allows
-        the one-launch decode, unless the context is set to the 4-launch path."""
+        the one-launch decode, unless the context is set to the several-launch path."""
         m = self.moe_cfg
         return ((m.hidden, m.inter, m.top_k, m.group) == (2048, 768, 8, 64) and m.n_exp <= 256
                 and bool(self.exe.paths() & OBS_PATH_FUSED_DECODE) and self.exe.decode_path != OBS_DECODE_MULTI)

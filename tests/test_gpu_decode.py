@@ -88,7 +88,7 @@ def test_moe_decode_with_post_attention_norm(exe, qwen_layer, path, seed):
 
 def test_moe_decode_fused_matches_multi_and_repeats(exe, qwen_layer):
     """Many back-to-back fused launches (device-side epoch advances every
-    launch) agree with the 4-launch path to bf16 rounding."""
+    launch) agree with the several-launch path to bf16 rounding."""
     t, layer, L = qwen_layer
     cfg = oh.MoeConfig(128, 8, 2048, 768, 64, True)
     rng = np.random.default_rng(1050)

@@ -5,7 +5,7 @@ No reference counterpart: the reference's executor setup (executor.rs:39-58)
 probes nothing, and its Metal dispatches never observe GPU errors. The
 outputs of the separate-launch paths are compared with the one-launch
 paths' on the same inputs (the items' arithmetic is the same, so the prefill
-results are bit-identical; the 4-launch decode is checked against its forced
+results are bit-identical; the several-launch decode is checked against its forced
 selection bit for bit and the oracle elsewhere).
 """
 import numpy as np

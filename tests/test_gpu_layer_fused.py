@@ -137,7 +137,7 @@ def test_layer_decode_graph_replay(exe, layer):
 
 def test_layer_decode_rejects_what_it_cannot_run(exe, layer):
     """A MoE layer without the post-attention norm, a shape outside the fused
-    decode's, misaligned caches and a context set to the 4-launch path are
+    decode's, misaligned caches and a context set to the several-launch path are
     refused before any launch."""
     attn, moe, cfg, kc, vt = layer
     r = _Run(exe, kc, vt)

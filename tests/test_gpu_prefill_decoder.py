@@ -180,7 +180,7 @@ def test_sdpa_prefill_rejects_bad_shapes(exe):
 
 
 # "split": 16 query heads, 8 experts, top-2 (the separate attention launches
-# and the 4-launch MoE path in the decode steps); "q30": the Qwen3-30B-A3B
+# and the several-launch MoE path in the decode steps); "q30": the Qwen3-30B-A3B
 # attention and expert shapes (32 / 4 heads, inter 768, top-8) with 16
 # experts, whose decode steps run the one-launch attention and MoE kernels.
 CFGS = {

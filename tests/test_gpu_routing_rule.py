@@ -4,7 +4,7 @@ The reference stores each router logit as a half (dequant_matvec_8bit.metal:30),
 runs the softmax and the top-k on those halves with ties to the lower id, and
 stores the weights as halves (moe_routing_topk.metal:24-56). The paths checked
 here: the standalone router (obs_q8_gate_logits + obs_route_topk), the fused
-one-launch decode, the four-launch decode and the prefill's computed routing.
+one-launch decode, the several-launch decode and the prefill's computed routing.
 
 Bars: logits, ids and weights bit-exact with the oracle (its router follows the
 kernels' documented logit reduction order and ORC_ROUTE_REF), on inputs built

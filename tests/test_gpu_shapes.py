@@ -3,7 +3,7 @@ widths the boundary accepts (forward.rs:421-441 decode, :164-247 prefill).
 
 * 256 experts takes the fused decode's four-slot routing variant; 64 experts
   leaves half of its two-slot key lanes absent.
-* hidden 4096 / inter 2048 is the widest decode shape (4-launch path).
+* hidden 4096 / inter 2048 is the widest decode shape (several-launch path).
 * prefill at 64 and 256 experts and at hidden 1024 / inter 512.
 
 Bars as elsewhere: routing ids and weights bit-exact with the oracle, layer

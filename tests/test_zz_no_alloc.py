@@ -3,7 +3,7 @@ intermediates live in a file-scope device array per GPU. Called through the C
 ABI (ctypes, no torch types) and compared with obs_moe_decode, which runs the
 same kernels on context-allocated workspaces: outputs, ids and weights must be
 identical bit for bit, on two calls in a row, the second with a smaller input
-(a smaller model shape, which takes the 4-launch path), then once more at the
+(a smaller model shape, which takes the several-launch path), then once more at the
 first shape (the fused path's exchange area keeps the earlier calls' epochs).
 """
 import ctypes as C
@@ -45,7 +45,7 @@ def _run(exe, fn, cfg, layer, x, res):
 def test_static_decode_equals_allocating_decode(exe):
     L = oh.lib()
     big = _case(exe, 3, 128, 2048, 768, 8, True)   # Qwen3-30B-A3B shape: the one-launch path
-    small = _case(exe, 4, 64, 1024, 512, 4, False)  # smaller input: the 4-launch path
+    small = _case(exe, 4, 64, 1024, 512, 4, False)  # smaller input: the several-launch path
     for case in (big, small, big):
         ref = _run(exe, L.obs_moe_decode, *case)
         got = _run(exe, L.obs_moe_decode_static, *case)
